@@ -14,7 +14,9 @@
 //    times zero, so the padded product equals the product);
 //  * C is computed into an M x N8 buffer when N % 8 != 0 and copied back to
 //    the caller's M x N rows.
-// Each element's sum runs over the same k as version 10's on the padded
+// Up to 128 rows with K >= 1024 go to f16_stream.hip instead, which reads B once
+// at any row alignment.
+// Through the copies each element's sum runs over the same k as version 10's on the padded
 // operands (the pad adds exact zeros), so the results are version 10's on
 // explicitly padded inputs, bit for bit.  The copies stream each operand
 // once more (at 4096 x 50257 x 4096: ~1.6 GB of copy traffic against ~1.7
@@ -120,7 +122,11 @@ hipError_t repitch(const void* src, void* dst, size_t rows, size_t width, size_t
 
 size_t out_bytes_of(vk_dtype d) { return d == VK_DTYPE_F16 ? 2 : 4; }
 
+// Few rows need no copies: f16_stream.hip reads B once at any row alignment.
+bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_stream_takes(m, n, k); }
+
 hipError_t launch_padded(const GemmArgs& a) {
+  if (few_rows(a.m, a.n, a.k)) return f16_stream_launch(a);
   const KernelEntry* inner = find_registered(kInnerVersion, VK_DTYPE_F16);
   if (!inner) return hipErrorInvalidValue;
   const PadLayout L = layout_of(a.m, a.n, a.k, a.num_cus, out_bytes_of(a.out_dtype));
@@ -155,7 +161,12 @@ hipError_t launch_padded(const GemmArgs& a) {
 
 // The workspace for an fp16 output; an fp32 output needs the larger C', so
 // the entry reports the fp32 size (both fit).
-size_t workspace_padded(size_t m, size_t n, size_t k, int num_cus) { return layout_of(m, n, k, num_cus, 4).total; }
+size_t workspace_padded(size_t m, size_t n, size_t k, int num_cus) {
+  return few_rows(m, n, k) ? f16_stream_workspace(m, n, k, num_cus) : layout_of(m, n, k, num_cus, 4).total;
+}
+
+// The two kinds of call keep different things at the workspace's start.
+int workspace_kind(size_t m, size_t n, size_t k) { return few_rows(m, n, k) ? 1 : 0; }
 
 // Version 10's limits on the padded problem.
 bool shape_ok_padded(size_t m, size_t n, size_t k) {
@@ -177,6 +188,7 @@ void register_f16_padded() {
   e.launch = launch_padded;
   e.workspace = workspace_padded;
   e.shape_ok = shape_ok_padded;
+  e.workspace_kind = workspace_kind;
   register_kernel(e);
 }
 

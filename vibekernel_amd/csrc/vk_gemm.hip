@@ -78,7 +78,8 @@ namespace {
 struct DeviceState {
   void* ws = nullptr;
   size_t ws_bytes = 0;
-  int ws_version = 0;  // version whose launch used the library workspace last (0: none)
+  const KernelEntry* ws_entry = nullptr;  // whose launch used the library workspace last (none: unknown)
+  int ws_kind = 0;                        // and in which of its layouts
   int num_cus = 0;
   void* scratch = nullptr;  // this device's copy of `scratch` (vk_gemm_noalloc)
 };
@@ -188,6 +189,7 @@ int run(int version, vk_dtype in, vk_dtype out, size_t m, size_t n, size_t k, co
   if (device_state(dev, &ds) != hipSuccess) return VK_ERR_HIP;
 
   const size_t need = e->workspace ? e->workspace(m, n, k, ds->num_cus) : 0;
+  const int kind = e->workspace_kind ? e->workspace_kind(m, n, k) : 0;
   bool ws_clean = false;
   bool owns_ws = false;  // this call uses the library workspace
   if (need > 0) {
@@ -206,17 +208,17 @@ int run(int version, vk_dtype in, vk_dtype out, size_t m, size_t n, size_t k, co
           ds->ws = nullptr;
           ds->ws_bytes = 0;
         }
-        ds->ws_version = 0;
+        ds->ws_entry = nullptr;
         if (hipMalloc(&ds->ws, need) != hipSuccess) return VK_ERR_HIP;
         ds->ws_bytes = need;
       }
       ws = ds->ws;
       ws_bytes = ds->ws_bytes;
-      ws_clean = ds->ws_version == version;
+      ws_clean = ds->ws_entry == e && ds->ws_kind == kind;
       // Until this launch is known to have been enqueued, the counters count
       // as unknown: a failed launch must not leave the next call skipping the
       // clear.
-      ds->ws_version = 0;
+      ds->ws_entry = nullptr;
       owns_ws = true;
     } else if (!ws || ws_bytes < need) {
       return VK_ERR_WORKSPACE;
@@ -242,7 +244,10 @@ int run(int version, vk_dtype in, vk_dtype out, size_t m, size_t n, size_t k, co
     // The kernels of a version leave the counters they use at zero, so the
     // next call of the same version may skip clearing them.
     std::lock_guard<std::mutex> lk(g_dev_mutex);
-    if (ds->ws == ws) ds->ws_version = version;
+    if (ds->ws == ws) {
+      ds->ws_entry = e;
+      ds->ws_kind = kind;
+    }
   }
   return VK_OK;
 }
@@ -334,7 +339,7 @@ int vk_gemm_release(void) {
     if (hipSetDevice(d) != hipSuccess || hipFree(vk::g_dev[d].ws) != hipSuccess) st = VK_ERR_HIP;
     vk::g_dev[d].ws = nullptr;
     vk::g_dev[d].ws_bytes = 0;
-    vk::g_dev[d].ws_version = 0;
+    vk::g_dev[d].ws_entry = nullptr;
   }
   if (hipSetDevice(cur) != hipSuccess) st = VK_ERR_HIP;
   return st;

@@ -21,8 +21,8 @@ struct GemmArgs {
   vk_dtype out_dtype;
   void* workspace;
   size_t workspace_bytes;
-  // True when the workspace is library-managed and was left by the previous
-  // call of this same version (counters it keeps are already reset); false
+  // True when the workspace is library-managed and was left by a call of this
+  // same version and workspace layout (counters it keeps are already reset); false
   // for a caller workspace or after (re)allocation or use by another version.
   bool workspace_clean;
   hipStream_t stream;
@@ -35,6 +35,8 @@ using LaunchFn = hipError_t (*)(const GemmArgs&);
 using WorkspaceFn = size_t (*)(size_t m, size_t n, size_t k, int num_cus);
 // Optional extra shape rule beyond the divisibility in caps (nullptr = none).
 using ShapeFn = bool (*)(size_t m, size_t n, size_t k);
+// Which of a version's workspace layouts a shape takes (nullptr: it has one).
+using KindFn = int (*)(size_t m, size_t n, size_t k);
 
 struct KernelEntry {
   int version;
@@ -44,6 +46,7 @@ struct KernelEntry {
   LaunchFn launch;
   WorkspaceFn workspace;  // nullptr: no workspace
   ShapeFn shape_ok;       // nullptr: caps only
+  KindFn workspace_kind;  // nullptr: one layout
 };
 
 void register_kernel(const KernelEntry& e);
@@ -51,6 +54,11 @@ void register_kernel(const KernelEntry& e);
 // The registered entry of a version (nullptr if none); for launchers that
 // run another version on a transformed problem.
 const KernelEntry* find_registered(int version, vk_dtype in);
+
+// fp16, few rows, any N >= 8 and K (f16_stream.hip).
+bool f16_stream_takes(size_t m, size_t n, size_t k);
+size_t f16_stream_workspace(size_t m, size_t n, size_t k, int num_cus);
+hipError_t f16_stream_launch(const GemmArgs& a);
 
 // Fill `words` 32-bit words with zero on `stream` (a kernel, not
 // hipMemsetAsync, so it may be captured into a graph).
