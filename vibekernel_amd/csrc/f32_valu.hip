@@ -3,25 +3,23 @@
 // The reference has the fp32 harness path (results/naive_cycle4/include/
 // playground/system.hpp:35-41, results/naive_fable_cycle2/src/CMakeLists.txt:5-11)
 // and its v0 ground truth (matmul_f32_v0_cblas.cpp:8-12) but no hand-written
-// fp32 kernel; its only GPU fp32 version called cublasSgemm.  Two
-// register-blocked VALU kernels share one tile and thread mapping:
-//   * 128x256 workgroup tile, BK = 16, 256 threads, 8x16 outputs per thread
-//     held as 4x4 register blocks (rows ty*4 and 64+ty*4, columns
-//     64*g + tx*4 for g = 0..3) so the LDS operand reads are 16-byte and
-//     conflict-free; one barrier per k-tile over two LDS buffers;
-//   * tile-divisible shapes: the k-loop as one asm block with hand-chosen
-//     registers, k-tiles staged by direct-to-LDS loads (f32_valu_asm_kernel);
-//   * any other shape: a C++ kernel with bounds checks, the next k-tile
-//     prefetched into registers and stored into LDS (A transposed, k-major);
-//     on grids of few 128x256 tiles the same kernel on 64x64 tiles (4x4
-//     outputs per thread) fills more CUs.
+// fp32 kernel; its only GPU fp32 version called cublasSgemm.  Every element is
+// one fused multiply-add per term, k ascending, in two forms:
+//   * tile-divisible shapes whose tiles fill the CUs: a register-blocked VALU
+//     kernel (f32_valu_asm_kernel), 128x256 workgroup tile, BK = 16, 256
+//     threads, 8x16 outputs per thread held as 4x4 register blocks (rows ty*4
+//     and 64+ty*4, columns 64*g + tx*4 for g = 0..3) so the LDS operand reads
+//     are 16-byte and conflict-free; one barrier per k-tile over two LDS
+//     buffers filled by direct-to-LDS loads; the k-loop is one asm block with
+//     hand-chosen registers;
+//   * any other shape: the same sums on the matrix cores (f32_any.hip).
 // Roofline: the VOP2 FMA (`v_fmac_f32_e32`) runs at the full 157.3 TFLOP/s
 // rate on MI355X (measured 146.7 on independent chains; the VOP3 form runs
 // at half), unless its three VGPR operands share a register bank, which
 // halves it.  The asm kernel's register layout rules that out: 106.0 TFLOP/s
-// at 4096^3 against 92.3 for the C++ kernel, where the compiler had put a
-// quarter of the FMAs' operands in one bank.  Both are power-limited (the
-// board at its ~1.4 kW cap, SCLK 1.9 GHz for the asm kernel).
+// at 4096^3 against 92.3 for a C++ form, where the compiler had put a quarter
+// of the FMAs' operands in one bank.  It is power-limited (the board at its
+// ~1.4 kW cap, SCLK 1.9 GHz).
 #include "vk_device.hpp"
 #include "vk_internal.hpp"
 
@@ -36,134 +34,6 @@ constexpr int kApitch = kTM + 4;     // As_t[k][m] row pitch (floats)
 constexpr int kLdA = kTM * kBK / 4 / 256;  // float4 loads of A per thread per k-tile
 constexpr int kLdB = kBK * kTN / 4 / 256;  // float4 loads of B per thread per k-tile
 static_assert(kLdA == 2 && kLdB == 4, "tile load mapping");
-
-// kRB row blocks of 64 and kNG column groups of 64 per tile, kKT-deep
-// k-tiles: 128x256x16 (the asm kernel's tile) or, for grids of few such
-// tiles, 64x64x32 (4x4 outputs per thread, 4 k-steps per unrolled loop body),
-// with the same per-element order.
-template <bool kCheck, int kRB = 2, int kNG = kCG, int kKT = vk::kBK>
-__global__ __launch_bounds__(256) void f32_valu_kernel(const float* __restrict__ A,
-                                                       const float* __restrict__ B,
-                                                       float* __restrict__ C, int64_t M, int64_t N,
-                                                       int64_t K) {
-  constexpr int kBK = kKT;  // k-tile depth
-  constexpr int kUnroll = kRB * kNG == 1 ? 4 : 2;  // k-steps per unrolled loop body
-  constexpr int kTM = 64 * kRB, kTN = 64 * kNG, kApitch = kTM + 4;
-  constexpr int kLdA = kTM * kBK / 4 / 256, kLdB = kBK * kTN / 4 / 256;
-  static_assert(kLdA * 1024 == kTM * kBK && kLdB * 1024 == kBK * kTN, "whole float4 loads per thread");
-  __shared__ __attribute__((aligned(16))) float As[2][kBK * kApitch];
-  __shared__ __attribute__((aligned(16))) float Bs[2][kBK * kTN];
-
-  const int tid = threadIdx.x;
-  const int tx = tid & 15, ty = tid >> 4;
-  const int64_t m0 = (int64_t)blockIdx.y * kTM;
-  const int64_t n0 = (int64_t)blockIdx.x * kTN;
-
-  // Global load mapping: A: TM rows x BK/4 float4 per row; B: BK rows x TN/4 float4.
-  constexpr int kC4A = kBK / 4;   // float4 per A row
-  constexpr int kC4B = kTN / 4;   // float4 per B row
-  float4v ra[kLdA], rb[kLdB];
-  auto load_tile = [&](int64_t k0) {
-#pragma unroll
-    for (int e = 0; e < kLdA; e++) {
-      const int idx = tid + 256 * e;
-      const int row = idx / kC4A, c4 = idx % kC4A;
-      const int64_t gr = m0 + row, gc = k0 + c4 * 4;
-      if (!kCheck) {
-        ra[e] = *reinterpret_cast<const float4v*>(&A[gr * K + gc]);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          ra[e][q] = (gr < M && gc + q < K) ? A[gr * K + gc + q] : 0.0f;
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < kLdB; e++) {
-      const int idx = tid + 256 * e;
-      const int krow = idx / kC4B, c4 = idx % kC4B;
-      const int64_t gr = k0 + krow, gc = n0 + c4 * 4;
-      if (!kCheck) {
-        rb[e] = *reinterpret_cast<const float4v*>(&B[gr * N + gc]);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          rb[e][q] = (gr < K && gc + q < N) ? B[gr * N + gc + q] : 0.0f;
-      }
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int e = 0; e < kLdA; e++) {
-      const int idx = tid + 256 * e;
-      const int row = idx / kC4A, c4 = idx % kC4A;
-#pragma unroll
-      for (int q = 0; q < 4; q++) As[buf][(c4 * 4 + q) * kApitch + row] = ra[e][q];
-    }
-#pragma unroll
-    for (int e = 0; e < kLdB; e++) {
-      const int idx = tid + 256 * e;
-      const int krow = idx / kC4B, c4 = idx % kC4B;
-      *reinterpret_cast<float4v*>(&Bs[buf][krow * kTN + c4 * 4]) = rb[e];
-    }
-  };
-
-  float acc[4 * kRB][4 * kNG];
-#pragma unroll
-  for (int i = 0; i < 4 * kRB; i++)
-#pragma unroll
-    for (int j = 0; j < 4 * kNG; j++) acc[i][j] = 0.0f;
-
-  const int64_t nk = (K + kBK - 1) / kBK;
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-  for (int64_t kt = 0; kt < nk; kt++) {
-    const int cur = (int)(kt & 1);
-    if (kt + 1 < nk) load_tile((kt + 1) * kBK);
-#pragma unroll kUnroll
-    for (int kk = 0; kk < kBK; kk++) {
-      float a[4 * kRB];
-#pragma unroll
-      for (int r = 0; r < kRB; r++) {
-        const float4v ar = *reinterpret_cast<const float4v*>(&As[cur][kk * kApitch + 64 * r + ty * 4]);
-#pragma unroll
-        for (int q = 0; q < 4; q++) a[4 * r + q] = ar[q];
-      }
-      float b[4 * kNG];
-#pragma unroll
-      for (int g = 0; g < kNG; g++) {
-        const float4v bg = *reinterpret_cast<const float4v*>(&Bs[cur][kk * kTN + 64 * g + tx * 4]);
-#pragma unroll
-        for (int q = 0; q < 4; q++) b[4 * g + q] = bg[q];
-      }
-#pragma unroll
-      for (int i = 0; i < 4 * kRB; i++)
-#pragma unroll
-        for (int j = 0; j < 4 * kNG; j++) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
-    }
-    if (kt + 1 < nk) {
-      store_tile(cur ^ 1);
-      __syncthreads();
-    }
-  }
-
-#pragma unroll
-  for (int i = 0; i < 4 * kRB; i++) {
-    const int64_t row = m0 + 64 * (i / 4) + ty * 4 + i % 4;
-#pragma unroll
-    for (int g = 0; g < kNG; g++) {
-      const int64_t col = n0 + g * 64 + tx * 4;
-      if (!kCheck) {
-        float4v v = {acc[i][g * 4 + 0], acc[i][g * 4 + 1], acc[i][g * 4 + 2], acc[i][g * 4 + 3]};
-        *reinterpret_cast<float4v*>(&C[row * N + col]) = v;
-      } else if (row < M) {
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (col + q < N) C[row * N + col + q] = acc[i][g * 4 + q];
-      }
-    }
-  }
-}
 
 // Every VGPR from v32 up: the registers the asm kernel below uses itself.
 #define VK_CLOBBER_V32_V255 \
@@ -428,43 +298,25 @@ __global__ __launch_bounds__(256) void f32_valu_asm_kernel(const float* __restri
 }
 #pragma clang diagnostic pop
 
-// 64x64 tiles where the 128x256 ones, eight times the work each, need more
-// rounds of the CUs for the same work (512^3: 8 tiles on 256 CUs).  Measured
-// (us per launch, 2 rounds, one box, against the 128x256 kernels): 512^3
-// 43.2 against 131.3, 1024^3 83.5 / 260.0, 1536^3 203.6 / 386.8, 2048^3
-// 376.2 / 514.7, 4096 x 1024 x 4096 737.4 / 1024.9; a 128x128 tile (8x8
-// outputs per thread) was slower than 64x64 on each of them (2048^3 420.5).
-// With one wave per SIMD the small tile waits on its loads and LDS reads:
-// 32-deep k-tiles and 4 k-steps per loop body took it further (512^3 35.5,
-// 1024^3 69.7, 2048^3 281.8; 48-deep 42.9 / 84.1 / 359.7, 32-deep with 2
-// k-steps per body 39.8 / 78.0 / 278.5, fully unrolled 37.5 / 78.8 /
-// 605.5).
-bool f32_valu_small(size_t m, size_t n, int num_cus) {
-  const int64_t c = num_cus > 0 ? num_cus : 1;
-  const int64_t big = (int64_t)((m + kTM - 1) / kTM) * (int64_t)((n + kTN - 1) / kTN);
-  const int64_t small = (int64_t)((m + 63) / 64) * (int64_t)((n + 63) / 64);
-  return 8 * ((big + c - 1) / c) > (small + c - 1) / c && (m + 63) / 64 <= 65535;
+// The asm kernel where its 128x256 tiles fill the CUs in as few rounds as
+// 64x64 tiles would (eight times the work each).
+bool fills_cus(size_t m, size_t n, int num_cus) {
+  const size_t c = num_cus > 0 ? num_cus : 1;
+  const size_t big = m / kTM * (n / kTN), small = (m + 63) / 64 * ((n + 63) / 64);
+  return 8 * ((big + c - 1) / c) <= (small + c - 1) / c;
 }
 
 hipError_t launch_f32(const GemmArgs& a) {
   const float* A = static_cast<const float*>(a.A);
   const float* B = static_cast<const float*>(a.B);
   float* C = static_cast<float*>(a.C);
-  if (f32_valu_small(a.m, a.n, a.num_cus)) {
-    hipLaunchKernelGGL((f32_valu_kernel<true, 1, 1, 32>), dim3((unsigned)((a.n + 63) / 64), (unsigned)((a.m + 63) / 64)),
-                       dim3(256), 0, a.stream, A, B, C, (int64_t)a.m, (int64_t)a.n, (int64_t)a.k);
-    return hipGetLastError();
-  }
-  dim3 grid((unsigned)((a.n + kTN - 1) / kTN), (unsigned)((a.m + kTM - 1) / kTM));
+  const size_t tiles_m = a.m / kTM, tiles_n = a.n / kTN;
   const bool full = a.m % kTM == 0 && a.n % kTN == 0 && a.k % kBK == 0 &&
                     ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0 &&
                     ((uintptr_t)C & 15) == 0 && asm_offsets_fit(a.m, a.n, a.k);
-  if (full)
-    hipLaunchKernelGGL(f32_valu_asm_kernel, dim3(grid.x * grid.y), dim3(256), 0, a.stream, A, B, C, (int)a.m,
-                       (int)a.n, (int)a.k);
-  else
-    hipLaunchKernelGGL(f32_valu_kernel<true>, grid, dim3(256), 0, a.stream, A, B, C, (int64_t)a.m,
-                       (int64_t)a.n, (int64_t)a.k);
+  if (!full || !fills_cus(a.m, a.n, a.num_cus)) return f32_any_launch(a);
+  hipLaunchKernelGGL(f32_valu_asm_kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, a.stream, A, B, C,
+                     (int)a.m, (int)a.n, (int)a.k);
   return hipGetLastError();
 }
 

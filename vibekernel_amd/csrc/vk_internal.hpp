@@ -55,6 +55,9 @@ void register_kernel(const KernelEntry& e);
 // run another version on a transformed problem.
 const KernelEntry* find_registered(int version, vk_dtype in);
 
+// fp32, any shape and alignment (f32_any.hip).
+hipError_t f32_any_launch(const GemmArgs& a);
+
 // fp16, few rows, any N >= 8 and K (f16_stream.hip).
 bool f16_stream_takes(size_t m, size_t n, size_t k);
 size_t f16_stream_workspace(size_t m, size_t n, size_t k, int num_cus);
