@@ -34,12 +34,13 @@
 // of K.
 // Measured (us per launch, fresh operands each, against the padded copies and
 // version 10): 4096 x 50257 weights at M = 1 / 32 (fp32 out) / 64 / 128 79.8 /
-// 92.3 / 110 / 191 against 311 / 318 / 316 / 326 (the streaming read alone is
-// 79.4); 16 x 8191 x 8192 31.9 against 127; 128 x 8191 x 8192 55.6 against 131;
-// 16 x 4095 x 4095 18.2 against 61.6; 64 x 1001 x 1025 15.8 against 33.5; 16 x
+// 92.2 / 110 / 191 against 311 / 318 / 316 / 326 (the streaming read alone is
+// 79.4); 16 x 8191 x 8192 29.5 against 127; 128 x 8191 x 8192 55.6 against 131;
+// 16 x 4095 x 4096 13.8 against 59; 64 x 1001 x 1025 15.5 against 33.5; 16 x
 // 301 x 16000 14.5 against 74.
 #include "vk_device.hpp"
 #include "vk_internal.hpp"
+#include "vk_stream.hpp"
 #include "vk_tile.hpp"
 
 #include <algorithm>
@@ -48,13 +49,11 @@
 namespace vk {
 namespace {
 
-constexpr int W = 4;                     // waves per workgroup
+constexpr int W = kStreamWaves;          // waves per workgroup
 constexpr int kThreads = 64 * W;
 constexpr int kKStep = 32;
 constexpr int kNC = 128;                 // columns per workgroup
 constexpr int kMaxRows = 128;
-constexpr int kMaxPieces = 32;
-constexpr size_t kCounterBytes = 4096;   // (column block, wave) counters
 
 typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(2)));
 typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -77,15 +76,15 @@ __device__ __forceinline__ uint32_t pack_halves(uint32_t first, uint32_t second)
   return __builtin_amdgcn_perm(second, first, kHi ? 0x07060302u : 0x05040100u);
 }
 
-__device__ __forceinline__ void store_row8(half_t* p, const float (&v)[8]) {
+__device__ __forceinline__ void store_row8(half_t* p, const float4v (&x)[2]) {
   half8 h;
 #pragma unroll
-  for (int c = 0; c < 8; c++) h[c] = convert_out<half_t>(v[c]);
+  for (int c = 0; c < 8; c++) h[c] = convert_out<half_t>(x[c / 4][c % 4]);
   *reinterpret_cast<uint4u*>(p) = __builtin_bit_cast(uint4v, h);
 }
-__device__ __forceinline__ void store_row8(float* p, const float (&v)[8]) {
-  *reinterpret_cast<float4u*>(p) = float4v{v[0], v[1], v[2], v[3]};
-  *reinterpret_cast<float4u*>(p + 4) = float4v{v[4], v[5], v[6], v[7]};
+__device__ __forceinline__ void store_row8(float* p, const float4v (&x)[2]) {
+  *reinterpret_cast<float4u*>(p) = x[0];
+  *reinterpret_cast<float4u*>(p + 4) = x[1];
 }
 
 template <int MB, typename OutT>
@@ -98,11 +97,12 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
   const int g = lane >> 4, i16 = lane & 15;
 
   const int ncb = (N + kNC - 1) / kNC;
-  // the row halves of a column block, which read the same B, and neighbouring
-  // column blocks, which share the cache lines at their edge, on one XCD
+  // the row halves of a column block, which read the same B, and a piece's
+  // neighbouring column blocks, which share the cache lines at their edge, on
+  // one XCD, a column block's pieces on different ones
   const int id = xcd_remap(blockIdx.x, ncb * ks * halves);
   const int piece = id / halves, m0 = (id - piece * halves) * (16 * MB);
-  const int cb = piece / ks, kp = piece - cb * ks;
+  const int kp = piece / ncb, cb = piece - kp * ncb;
   const int slot0 = (cb * halves + (m0 ? 1 : 0)) * ks;  // this block's first partial slot
   const int n0 = cb * kNC;
   const int parts = ks * W, p = kp * W + wave;
@@ -202,111 +202,11 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
     multiply(s);
   }
 
-  // Two row blocks at a time through LDS: per wave 16 pieces of 1 KB
-  // (2 blocks x 4 rows x 2 halves of 8 columns, 16 bytes per lane); wave q
-  // keeps row 4g + q of each block.
-  constexpr int kPair = 2;
-  __shared__ float4v lds[W][kPair * 8][64];
-  float4v red[MB][2];
-#pragma unroll
-  for (int r0 = 0; r0 < MB; r0 += kPair) {
-    if (r0) __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kPair; i++)
-      if (r0 + i < MB)
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-#pragma unroll
-          for (int h = 0; h < 2; h++)
-            lds[wave][(i * 4 + e) * 2 + h][lane] = float4v{acc[r0 + i][4 * h][e], acc[r0 + i][4 * h + 1][e],
-                                                           acc[r0 + i][4 * h + 2][e], acc[r0 + i][4 * h + 3][e]};
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kPair; i++)
-      if (r0 + i < MB)
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-          float4v t = lds[0][(i * 4 + wave) * 2 + h][lane];
-#pragma unroll
-          for (int w = 1; w < W; w++) t += lds[w][(i * 4 + wave) * 2 + h][lane];
-          red[r0 + i][h] = t;
-        }
-  }
-  auto store_c = [&](int r, const float4v (&x)[2]) {
-    const int row = m0 + 16 * r + 4 * g + wave;
-    const float v[8] = {x[0][0], x[0][1], x[0][2], x[0][3], x[1][0], x[1][1], x[1][2], x[1][3]};
-    if (row < M) store_row8(C + (size_t)row * N + col, v);
-  };
-  if (ks == 1) {
-#pragma unroll
-    for (int r = 0; r < MB; r++) store_c(r, red[r]);
-    return;
-  }
-  // K split over workgroups, as in f16_skinny_wk.hip: slot (column
-  // block, half, piece) holds 4 wave regions of 2 MB KB; a wave that finds every other piece in
-  // memory is the last and sums them in k order, its own from registers.
-  constexpr uint32_t kWaveRegion = MB * 2048;
-  constexpr uint32_t kSlotBytes = W * kWaveRegion;
-  const __amdgpu_buffer_rsrc_t prs =
-      __builtin_amdgcn_make_buffer_rsrc(part, 0, (int)((uint32_t)(ncb * ks * halves) * kSlotBytes), kBufferWord3);
-  auto soff = [&](int q) { return (uint32_t)(slot0 + q) * kSlotBytes + (uint32_t)wave * kWaveRegion; };
-  const uint32_t vlane = (uint32_t)lane * 16;
-  unsigned* cnt = counters + slot0 / ks * W + wave;
-  const unsigned seen =
-      __builtin_amdgcn_readfirstlane(__hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-  if (seen != (unsigned)(ks - 1)) {
-#pragma unroll
-    for (int r = 0; r < MB; r++)
-#pragma unroll
-      for (int h = 0; h < 2; h++) store_partial(prs, vlane + (2 * r + h) * 1024, soff(kp), red[r][h]);
-    wait_vmcnt0_ordered();  // the partial is in memory before the counter moves
-    unsigned old = 0;
-    if (lane == 0) old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (__builtin_amdgcn_readfirstlane(old) != (unsigned)(ks - 1)) return;
-  }
-  asm volatile("" ::: "memory");  // the other pieces are read after the counter
-  // P pieces of RB row blocks at a time (up to 32 loads in flight); a piece
-  // past ks reads the last one's slot and is not added.
-  auto fold = [&](auto pieces) {
-    constexpr int P = decltype(pieces)::value;
-    constexpr int RB = 16 / P < MB ? 16 / P : MB;
-#pragma unroll
-    for (int r0 = 0; r0 < MB; r0 += RB) {
-      float4v t[RB][2];
-      for (int q0 = 0; q0 < ks; q0 += P) {
-        float4v x[P][RB][2];
-#pragma unroll
-        for (int q = 0; q < P; q++)
-#pragma unroll
-          for (int i = 0; i < RB; i++)
-#pragma unroll
-            for (int h = 0; h < 2; h++)
-              if (r0 + i < MB)
-                x[q][i][h] = load_partial(prs, vlane + (2 * (r0 + i) + h) * 1024, soff(min(q0 + q, ks - 1)));
-#pragma unroll
-        for (int q = 0; q < P; q++)
-          if (q0 + q < ks)
-#pragma unroll
-            for (int i = 0; i < RB; i++)
-#pragma unroll
-              for (int h = 0; h < 2; h++)
-                if (r0 + i < MB) {
-                  const float4v v = q0 + q == kp ? red[r0 + i][h] : x[q][i][h];
-                  t[i][h] = q0 + q == 0 ? v : t[i][h] + v;
-                }
-      }
-#pragma unroll
-      for (int i = 0; i < RB; i++)
-        if (r0 + i < MB) store_c(r0 + i, t[i]);
-    }
-  };
-  if (ks == 2)
-    fold(std::integral_constant<int, 2>{});
-  else if (ks == 4)
-    fold(std::integral_constant<int, 4>{});
-  else
-    fold(std::integral_constant<int, 8>{});
-  if (lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  stream_finish<MB, 2>(acc, lane, wave, ks, kp, slot0, ncb * halves * ks, part, counters,
+                       [&](int r, const float4v (&x)[2]) {
+                         const int row = m0 + 16 * r + 4 * g + wave;
+                         if (row < M) store_row8(C + (size_t)row * N + col, x);
+                       });
 }
 
 // Up to 64 rows a workgroup takes them all; more are cut in two halves of
@@ -316,14 +216,8 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
 int halves_of(size_t m) { return m > 64 ? 2 : 1; }
 int blocks_of(size_t m) { return (int)(((m + 15) / 16 + halves_of(m) - 1) / halves_of(m)); }
 
-// Workgroups per column block and half: doubled while the grid stays within
-// one per CU and every wave keeps at least 4 k-steps.
 int pieces_of(size_t m, size_t n, size_t k, int num_cus) {
-  const size_t steps = k / kKStep, blocks = (n + kNC - 1) / kNC * halves_of(m);
-  int ks = 1;
-  if (blocks * W * sizeof(unsigned) > kCounterBytes) return 1;
-  while (ks < kMaxPieces && blocks * ks * 2 <= (size_t)num_cus && steps / (ks * 2) >= 4 * W) ks *= 2;
-  return ks;
+  return stream_pieces((n + kNC - 1) / kNC * halves_of(m), k / kKStep, num_cus);
 }
 
 template <int MB, typename OutT>
@@ -331,14 +225,8 @@ hipError_t launch_t(const GemmArgs& a) {
   const int ks = pieces_of(a.m, a.n, a.k, a.num_cus), halves = halves_of(a.m);
   unsigned* counters = nullptr;
   float* part = nullptr;
-  if (ks > 1) {
-    counters = static_cast<unsigned*>(a.workspace);
-    part = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + kCounterBytes);
-    if (!a.workspace_clean) {
-      const hipError_t e = zero_words(counters, kCounterBytes / 4, a.stream);
-      if (e != hipSuccess) return e;
-    }
-  }
+  const hipError_t e = stream_buffers(a, ks, counters, part);
+  if (e != hipSuccess) return e;
   const unsigned grid = (unsigned)((a.n + kNC - 1) / kNC * ks * halves);
   hipLaunchKernelGGL((f16_stream_kernel<MB, OutT>), dim3(grid), dim3(kThreads), 0, a.stream,
                      static_cast<const half_t*>(a.A), static_cast<const half_t*>(a.B), static_cast<OutT*>(a.C),
@@ -361,8 +249,7 @@ bool f16_stream_takes(size_t m, size_t n, size_t k) {
 
 size_t f16_stream_workspace(size_t m, size_t n, size_t k, int num_cus) {
   const int ks = pieces_of(m, n, k, num_cus);
-  if (ks == 1) return 0;
-  return kCounterBytes + (n + kNC - 1) / kNC * ks * halves_of(m) * W * (size_t)blocks_of(m) * 2048;
+  return stream_workspace((n + kNC - 1) / kNC * halves_of(m), ks, blocks_of(m), 2);
 }
 
 hipError_t f16_stream_launch(const GemmArgs& a) {

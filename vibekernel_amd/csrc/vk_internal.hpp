@@ -58,6 +58,11 @@ const KernelEntry* find_registered(int version, vk_dtype in);
 // fp32, any shape and alignment (f32_any.hip).
 hipError_t f32_any_launch(const GemmArgs& a);
 
+// fp32, few rows, N and K multiples of 4 (f32_stream.hip).
+bool f32_stream_takes(size_t m, size_t n, size_t k);
+size_t f32_stream_workspace(size_t m, size_t n, size_t k, int num_cus);
+hipError_t f32_stream_launch(const GemmArgs& a);
+
 // fp16, few rows, any N >= 8 and K (f16_stream.hip).
 bool f16_stream_takes(size_t m, size_t n, size_t k);
 size_t f16_stream_workspace(size_t m, size_t n, size_t k, int num_cus);
