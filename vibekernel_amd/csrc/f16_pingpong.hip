@@ -612,6 +612,22 @@ static_assert(lds_bytes_of<kAblB2>() >= 8 * 128 * 64 * 2, "fp16 epilogue staging
 template <typename OutT>
 struct Epi16;
 
+// 16 bytes of a row of C that has `left` elements from there on.
+typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(2)));
+template <typename OutT>
+__device__ __forceinline__ void store_chunk(OutT* p, const uint4v& v, int left) {
+  constexpr int kE = 16 / sizeof(OutT);
+  if (left >= kE) {
+    *reinterpret_cast<uint4u*>(p) = v;
+  } else if (left > 0) {
+    OutT x[kE];
+    __builtin_memcpy(x, &v, 16);
+#pragma unroll
+    for (int e = 0; e < kE - 1; e++)
+      if (e < left) p[e] = x[e];
+  }
+}
+
 // fp16: the whole 128x64 block fits the region (row pitch 128 B, see
 // epi16_unit_addr), so only the second flush() stores, 8 rows x 8 chunks per
 // read.
@@ -634,12 +650,12 @@ struct Epi16<half_t> {
     }
   }
   // The same for a block at (row0, col0) of C that may reach past M rows or
-  // N columns (N a multiple of 8): chunks outside are not stored.
+  // N columns, which are not stored; rows of C start on any 2-byte boundary.
   static __device__ __forceinline__ void flush_edge(uint32_t wbase, half_t* C, int M, int N, int row0, int col0,
                                                     int lane, int half) {
     if (half == 0) return;
     const int rsub = lane >> 3, ch = lane & 7;
-    const bool col_in = col0 + ch * 8 < N;
+    const int left = N - (col0 + ch * 8);  // columns from this lane's chunk on
     // Plain stores on the edge paths (version 10, the split tails with
     // edges): the sc1 stores that help the whole tiles made the 128 x 128
     // kernel's edge path slower at 1000^3.
@@ -647,7 +663,7 @@ struct Epi16<half_t> {
     for (int q = 0; q < 16; q++) {
       const int row = 8 * q + rsub;
       const uint4v v = epi16_read_pair(wbase, row, ch);
-      if (col_in && row0 + row < M) *reinterpret_cast<uint4v*>(C + (size_t)(row0 + row) * N + col0 + ch * 8) = v;
+      if (row0 + row < M) store_chunk(C + (size_t)(row0 + row) * N + col0 + ch * 8, v, left);
     }
   }
 };
@@ -675,13 +691,13 @@ struct Epi16<float> {
   static __device__ __forceinline__ void flush_edge(uint32_t wbase, float* C, int M, int N, int row0, int col0,
                                                     int lane, int half) {
     const int rsub = lane >> 4, ch = lane & 15;
-    const bool col_in = col0 + ch * 4 < N;
+    const int left = N - (col0 + ch * 4);
 #pragma unroll
     for (int q = 0; q < 16; q++) {
       const int row = 4 * q + rsub;
       const uint4v v = lds_read16(wbase + row * 256 + 16 * (ch ^ (row & 15)));
       const int r = row0 + half * 64 + row;
-      if (col_in && r < M) *reinterpret_cast<uint4v*>(C + (size_t)r * N + col0 + ch * 4) = v;
+      if (r < M) store_chunk(C + (size_t)r * N + col0 + ch * 4, v, left);
     }
     if (half == 0) wait_lgkmcnt0();
   }
@@ -1146,7 +1162,7 @@ hipError_t launch_abl(const GemmArgs& a) {
 template <typename OutT>
 __global__ __launch_bounds__(kThreads) void f16_pp16_edge_kernel(const half_t* __restrict__ A,
                                                                  const half_t* __restrict__ B,
-                                                                 OutT* __restrict__ C, int M, int N, int K) {
+                                                                 OutT* __restrict__ C, int M, int N, int K, int ldc) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1160,7 +1176,7 @@ __global__ __launch_bounds__(kThreads) void f16_pp16_edge_kernel(const half_t* _
 
   float4v acc[8][4];
   pp16_mainloop<true>(A, B, N, K, m0, n0, 0, (K + kBK - 1) / kBK, lds_base, grp, gw, lane, acc, M);
-  epilogue16_edge<OutT>(acc, lds_base + wave * (128 * 64 * 2), C, M, N, m0 + grp * 128, n0 + gw * 64,
+  epilogue16_edge<OutT>(acc, lds_base + wave * (128 * 64 * 2), C, M, ldc, m0 + grp * 128, n0 + gw * 64,
                         lane_from_exec());
 }
 
@@ -1173,7 +1189,7 @@ hipError_t launch_edge_t(const GemmArgs& a) {
   const int tiles = (int)(((a.m + kBM - 1) / kBM) * ((a.n + kBN - 1) / kBN));
   hipLaunchKernelGGL(kfn, dim3(tiles), dim3(kThreads), kLdsBytes, a.stream,
                      static_cast<const half_t*>(a.A), static_cast<const half_t*>(a.B),
-                     static_cast<OutT*>(a.C), (int)a.m, (int)a.n, (int)a.k);
+                     static_cast<OutT*>(a.C), (int)a.m, (int)a.n, (int)a.k, (int)(a.ldc ? a.ldc : a.n));
   return hipGetLastError();
 }
 
@@ -1291,7 +1307,7 @@ template <typename OutT, bool kEdge>
 __global__ __launch_bounds__(kThreads) void f16_pp16_sk_kernel(const half_t* __restrict__ A,
                                                                const half_t* __restrict__ B,
                                                                OutT* __restrict__ C, int M, int N, int K, int dp,
-                                                               int units, int pieces, int chunks,
+                                                               int units, int pieces, int chunks, int ldc,
                                                                float* __restrict__ part,
                                                                unsigned* __restrict__ counters) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -1324,7 +1340,8 @@ __global__ __launch_bounds__(kThreads) void f16_pp16_sk_kernel(const half_t* __r
   };
   unsigned* cnt = counters + (size_t)w.tile * kSkWaves + wave;
   if (w.np == 1 || sk_arrive(acc, w.np, w.p, prsrc, part_off, cnt))
-    sk_write_c<OutT, kEdge>(acc, w.np, w.p, prsrc, part_off, cnt, wstage, C, M, N, m0 + grp * 128, n0 + gw * 64);
+    sk_write_c<OutT, kEdge>(acc, w.np, w.p, prsrc, part_off, cnt, wstage, C, M, kEdge ? ldc : N, m0 + grp * 128,
+                             n0 + gw * 64);
 }
 
 // Split-tail plan of a shape: kEdge counts the tiles and k-tiles that reach
@@ -1354,7 +1371,7 @@ hipError_t launch_sk_t(const GemmArgs& a) {
   }
   hipLaunchKernelGGL(kfn, dim3((unsigned)(p.dp + p.units)), dim3(kThreads), kLdsBytes, a.stream,
                      static_cast<const half_t*>(a.A), static_cast<const half_t*>(a.B), static_cast<OutT*>(a.C),
-                     (int)a.m, (int)a.n, (int)a.k, p.dp, p.units, p.pieces, p.chunks, part, counters);
+                     (int)a.m, (int)a.n, (int)a.k, p.dp, p.units, p.pieces, p.chunks, (int)(a.ldc ? a.ldc : a.n), part, counters);
   return hipGetLastError();
 }
 

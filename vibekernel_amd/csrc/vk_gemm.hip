@@ -47,7 +47,7 @@ std::once_flag g_init_once;
 
 void init_registry() {
   std::call_once(g_init_once, [] {
-    register_f16_simple();
+    register_f16_any();
     register_f16_dma();
     register_f16_skinny();
     register_f16_pingpong();
@@ -239,6 +239,7 @@ int run(int version, vk_dtype in, vk_dtype out, size_t m, size_t n, size_t k, co
   a.stream = s;
   a.device = dev;
   a.num_cus = ds->num_cus;
+  a.ldc = 0;
   if (e->launch(a) != hipSuccess) return VK_ERR_HIP;
   if (owns_ws) {
     // The kernels of a version leave the counters they use at zero, so the

@@ -28,6 +28,9 @@ struct GemmArgs {
   hipStream_t stream;
   int device;
   int num_cus;
+  // Row pitch of C and its columns, where B has more (version 10 on a B whose
+  // rows are padded to n columns); 0: n.
+  size_t ldc;
 };
 
 using LaunchFn = hipError_t (*)(const GemmArgs&);
@@ -63,6 +66,9 @@ bool f32_stream_takes(size_t m, size_t n, size_t k);
 size_t f32_stream_workspace(size_t m, size_t n, size_t k, int num_cus);
 hipError_t f32_stream_launch(const GemmArgs& a);
 
+// fp16, any shape and alignment (f16_any.hip).
+hipError_t f16_any_launch(const GemmArgs& a);
+
 // fp16, few rows, any N >= 8 and K (f16_stream.hip).
 bool f16_stream_takes(size_t m, size_t n, size_t k);
 size_t f16_stream_workspace(size_t m, size_t n, size_t k, int num_cus);
@@ -73,7 +79,7 @@ hipError_t f16_stream_launch(const GemmArgs& a);
 hipError_t zero_words(void* p, size_t words, hipStream_t stream);
 
 // Per-translation-unit registration hooks (called once from vk_gemm.hip).
-void register_f16_simple();
+void register_f16_any();
 void register_f16_dma();
 void register_f16_skinny();
 void register_f16_pingpong();
