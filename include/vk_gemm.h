@@ -153,6 +153,12 @@ int vk_gemm_list(vk_dtype in_dtype, int* out, int max_count);
 int vk_gemm_check(int version, vk_dtype in_dtype, vk_dtype out_dtype, size_t m, size_t n, size_t k,
                   const void* A, const void* B, const void* C);
 
+/* The fastest version that accepts this shape with 4 KiB-aligned operands on
+ * the current device (with no device to ask, an MI355X's 256 CUs are assumed),
+ * or VK_ERR_SHAPE if none does.  Launches nothing.  The reference picks
+ * versions at build time only (CMakeLists.txt MATMUL_VERSION). */
+int vk_gemm_pick(vk_dtype in_dtype, vk_dtype out_dtype, size_t m, size_t n, size_t k);
+
 /* Free library-managed workspaces on every device. */
 int vk_gemm_release(void);
 

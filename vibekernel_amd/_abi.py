@@ -39,6 +39,7 @@ EXPORTED_SYMBOLS = (
     "vk_gemm_query",
     "vk_gemm_list",
     "vk_gemm_check",
+    "vk_gemm_pick",
     "vk_gemm_release",
     "vk_status_string",
     "vk_gemm_abi_version",
@@ -132,6 +133,8 @@ def load() -> ctypes.CDLL:
     L.vk_gemm_list.restype = ci
     L.vk_gemm_check.argtypes = [ci, ci, ci, sz, sz, sz, vp, vp, vp]
     L.vk_gemm_check.restype = ci
+    L.vk_gemm_pick.argtypes = [ci, ci, sz, sz, sz]
+    L.vk_gemm_pick.restype = ci
     L.vk_gemm_release.argtypes = []
     L.vk_gemm_release.restype = ci
     L.vk_status_string.argtypes = [ci]
@@ -194,8 +197,12 @@ def check(version, in_dtype, out_dtype, m, n, k, a_ptr, b_ptr, c_ptr) -> int:
     return int(load().vk_gemm_check(version, in_dtype, out_dtype, m, n, k, a_ptr, b_ptr, c_ptr))
 
 
+def pick(in_dtype, out_dtype, m, n, k) -> int:
+    return load().vk_gemm_pick(in_dtype, out_dtype, m, n, k)
+
+
 def gemm(version, in_dtype, out_dtype, m, n, k, a_ptr, b_ptr, c_ptr, stream=None) -> int:
-    return int(load().vk_gemm(version, in_dtype, out_dtype, m, n, k, a_ptr, b_ptr, c_ptr, stream))
+    return load().vk_gemm(version, in_dtype, out_dtype, m, n, k, a_ptr, b_ptr, c_ptr, stream)
 
 
 def gemm_ws(version, in_dtype, out_dtype, m, n, k, a_ptr, b_ptr, c_ptr, ws_ptr, ws_bytes,

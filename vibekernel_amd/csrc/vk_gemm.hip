@@ -103,6 +103,14 @@ hipError_t device_state(int dev, DeviceState** out) {
   return hipSuccess;
 }
 
+// Compute units of the current device (plans depend on them); with no device
+// to ask, an MI355X's 256 are assumed.
+int cus_or_default() {
+  int dev = 0;
+  DeviceState* ds = nullptr;
+  return hipGetDevice(&dev) == hipSuccess && device_state(dev, &ds) == hipSuccess ? ds->num_cus : 256;
+}
+
 // Device address of this device's copy of `scratch`, looked up once per
 // device with that device current.
 hipError_t scratch_of(int dev, void** out) {
@@ -253,6 +261,109 @@ int run(int version, vk_dtype in, vk_dtype out, size_t m, size_t n, size_t k, co
   return VK_OK;
 }
 
+// ---- the version for a shape ----
+// The fastest version that accepts this shape (checked with vk_gemm_check
+// on 4 KiB-aligned placeholder addresses; nothing is launched): for fp16
+// the skinny kernels up to M = 128 (version 14 where it suits, else version
+// 8; version 4 up to 64) and version 8 from 129 to 255 rows where version 11
+// does not suit, then the
+// 128 x 128 tiles of version 11 where they suit the grid, then the 256x256 kernels
+// (fastest first; version 10 takes shapes off the 256 x 256 x 64 grid
+// whose N and K are multiples of 8), then version 15 (N or K off the multiples
+// of 8, from M N K = 2^24 on), then the any-shape kernel.  Version 11
+// is taken, with T its 128 x 128 tiles on C compute units:
+//   * on the 256 x 256 x 64 grid, where T <= C (one wave; with 2 T <= C it
+//   splits K over the idle CUs itself).  Measured on MI355X, us per
+//   launch against version 9's split tail: 1024 x 4096 x 4096 33.6
+//   against 46.2 (version 7: 64.5), 1024 x 1024 x 8192 29.1 against
+//   43.9, 512 x 512 x 8192 19.7 against 41.7, 512 x 4096 x 4096 24.7
+//   against 35.1; beyond one wave 1536 x 4096 x 4096 (T = 384) took 58.7
+//   against 50.6;
+//   * off it, where T <= 3 C / 2 (version 10, whose split pieces do not stay
+//   on one XCD there and whose edge tiles are twice as wide, measured
+//   slower on every such shape: 1000 x 1000 x 1000 23.0 us against 9.8,
+//   2000 x 3000 x 1000 (T = 384) 25.2 against 21.2, 1000 x 1000 x 4000
+//   (T = 64) 36.6 against 23.0).
+// From M = 129 version 11 also beats the skinny split-K version 8 wherever
+// it is taken (us per launch, one box: 192 x 4096 x 4096 22.5 against
+// 30.2, 192 x 8192 x 8192 39.8 against 46.0, 192 x 14336 x 4096 32.9
+// against 42.4, 256 x 8192 x 8192 39.8 against 55.6; another box, v11
+// against v8 at N x K = 4096 x 4096 / 4096 x 8192 / 8192 x 4096 / 8192 x
+// 8192 / 14336 x 4096 / 4096 x 14336: M = 136 21.1 / 27.1 / 24.1 / 37.1 /
+// 28.9 / 37.9 against 25.9 / 31.5 / 27.0 / 37.4 / 32.8 / 39.4; M = 160
+// 21.1 / 27.8 / 24.5 / 39.0 / 31.1 / 39.5 against 26.2 / 31.9 / 27.6 /
+// 38.5 / 33.8 / 39.8; M = 184 21.9 / 28.3 / 24.8 / 39.8 / 32.6 / 38.9
+// against 30.3 / 38.7 / 32.5 / 45.6 / 41.1 / 46.9).
+// Version 14 (K split over the waves of a workgroup, 64-column blocks) is
+// taken up to M = 64 where 2048 < N <= 4096 (but not up to M = 32 with
+// K > 12288) and up to M = 8 where 1024 < N <= 2048 and K <= 8192, and
+// from M = 65 to 128 where N <= 4096 and K <= 8192.  Against version 8
+// (us per launch, one box): M = 72 / 96 / 128 at N x K = 4096 x 6144
+// 16.8 / 19.3 / 22.9 against 20.2 / 22.6 / 25.0, at 4096 x 8192 19.2 /
+// 22.2 / 26.6 against 22.7 / 24.3 / 27.7, at 2048 x 8192 16.5 / 18.2 /
+// 21.5 against 18.9 / 20.5 / 24.1, at 3072 x 6144 17.4 / 19.5 / 23.1
+// against 18.3 / 20.0 / 22.9; at K = 11264 mixed (4096 columns: 23.7 /
+// 27.9 / 34.2 against 26.7 / 28.3 / 31.3); M = 1 / 4 / 8 at N x K = 1536 x
+// 8192 8.6 / 9.0 / 9.2 against 10.0 / 10.2 / 10.3, 2048 x 8192 9.6 / 10.1
+// / 10.6 against 10.4 / 10.7 / 10.7, 2048 x 4096 8.7 / 9.0 / 9.2 against
+// 8.9 / 9.1 / 9.2, but 2048 x 14336 16.0 / 16.5 / 16.4 against 15.7 /
+// 15.9 / 16.0 and M = 16 at N = 2048 (K = 4096 / 8192 / 14336: 9.3 / 11.1
+// / 16.4 against 9.1 / 10.8 / 16.0).  At K = 14336, N = 4096 version 8 is faster up
+// to M = 32 (us per launch against version 14, 2 rounds on one box: M = 1
+// 22.3 against 22.6, 16 22.5 against 23.6, 32 23.8 against 24.1; N =
+// 3072, M = 16 19.1 against 20.1; N = 2560, M = 16 17.8 against 18.0) and
+// version 14 from M = 48 (26.1 against 25.4; M = 64 28.4 against 27.2);
+// at K = 11264 they are within 2 % (M = 16 19.4 / 19.8, M = 1 19.1 /
+// 18.9) and at K = 8192 version 14 wins (M = 1 16.4 / 15.5, 16 16.9 /
+// 16.0, 32 18.4 / 16.5).  Measured on MI355X
+// against version 8 (us per launch, one box, M = 1 / 16 / 64 / 128):
+// N = 4096, K = 4096 8.1 / 9.1 / 14.4 / 18.4 against 9.5 / 9.9 / 16.2 /
+// 21.8; N = 3072, K = 2048 7.2 / 7.6 / 11.6 / 14.4 against 8.1 / 8.3 /
+// 13.5 / 20.3; N = 4096, K = 14336 22.1 / 22.9 / 27.1 / 39.0 against
+// 22.2 / 22.5 / 28.5 / 35.3; N = 2048, K = 8192 at M = 128 21.0 against
+// 23.4, at M = 16 10.2 against 10.5; N = 1024, K = 2048 8.3 / 8.6 / 12.4 /
+// 15.9 against 6.7 / 7.0 / 10.9 / 17.6.  Every 64 columns re-read all of
+// A (at M = 128 twice B's bytes), which costs it at large M and K; from
+// N = 5120 its power-of-two K split also leaves CUs idle (80 column blocks
+// x 2): 128 x 8192 x 8192 41.8 against 32.9.
+// The split-tail version 9 comes first among the 256x256 kernels only where
+// its schedule splits tiles on this device (it then needs a workspace);
+// elsewhere it would run version 7's whole tiles.  The reference picks
+// versions at build time only (CMakeLists.txt MATMUL_VERSION); this is a
+// convenience.
+int pick(vk_dtype in, vk_dtype out, size_t m, size_t n, size_t k) {
+  static constexpr int kOrderF16[] = {14, 8, 4, 11, 9, 7, 10, 6, 5, 3, 2, 15, 1};
+  static constexpr int kOrderF32[] = {2, 3, 1};
+  const void* at = reinterpret_cast<const void*>(uintptr_t{4096});
+  auto takes = [&](int v) { return validate(find(v, in), out, m, n, k, at, at, at) == VK_OK; };
+  if (in != VK_DTYPE_F16) {
+    for (int v : kOrderF32)
+      if (takes(v)) return v;
+    return VK_ERR_SHAPE;
+  }
+  const size_t lim = 0x7fffffffu;  // no version takes more (and the counts below stay within 64 bits)
+  if (m > lim || n > lim || k > lim) return VK_ERR_SHAPE;
+
+  const int cus = cus_or_default();
+  const size_t tiles = (m + 127) / 128 * ((n + 127) / 128);
+  const bool v11_suits =
+      m % 256 == 0 && n % 256 == 0 && k % 64 == 0 ? tiles <= (size_t)cus : 2 * tiles <= 3 * (size_t)cus;
+  bool v14_suits = m <= 128 && n <= 4096 && !(m <= 32 && k > 12288);
+  if (v14_suits) v14_suits = m <= 64 ? n > 2048 || (m <= 8 && n > 1024 && k <= 8192) : k <= 8192;
+  const bool v15_suits = (unsigned __int128)m * n * k >= (1u << 24);  // below: version 1
+
+  for (int v : kOrderF16) {
+    if (v == 14 && !v14_suits) continue;
+    if (v == 8 && m > 128 && v11_suits && takes(11)) continue;
+    if (v == 11 && !v11_suits) continue;
+    if (v == 15 && !v15_suits) continue;
+    if (!takes(v)) continue;
+    if (v == 9 && find(9, in)->workspace(m, n, k, cus) == 0) continue;
+    return v;
+  }
+  return VK_ERR_SHAPE;
+}
+
 }  // namespace
 
 void register_kernel(const KernelEntry& e) {
@@ -294,12 +405,11 @@ int vk_gemm_noalloc(int version, vk_dtype in_dtype, vk_dtype out_dtype, size_t m
 size_t vk_gemm_workspace_bytes(int version, vk_dtype in_dtype, size_t m, size_t n, size_t k) {
   const vk::KernelEntry* e = vk::find(version, in_dtype);
   if (!e || !e->workspace) return 0;
-  // The split-tail schedule depends on the current device's compute-unit count;
-  // with no device to ask, an MI355X (256 CUs) is assumed.
-  int cus = 256, dev = 0;
-  vk::DeviceState* ds = nullptr;
-  if (hipGetDevice(&dev) == hipSuccess && vk::device_state(dev, &ds) == hipSuccess) cus = ds->num_cus;
-  return e->workspace(m, n, k, cus);
+  return e->workspace(m, n, k, vk::cus_or_default());
+}
+
+int vk_gemm_pick(vk_dtype in_dtype, vk_dtype out_dtype, size_t m, size_t n, size_t k) {
+  return vk::pick(in_dtype, out_dtype, m, n, k);
 }
 
 const char* vk_gemm_name(int version, vk_dtype in_dtype) {
