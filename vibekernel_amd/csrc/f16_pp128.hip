@@ -558,8 +558,26 @@ hipError_t launch_out(const GemmArgs& a) {
   return grid ? launch_t<OutT, false, false>(a, p) : launch_t<OutT, true, false>(a, p);
 }
 
+// A grid of 128 x 128 tiles just past a whole number of rounds of the CUs (258
+// on 256) leaves most of its last round empty; where the 64-row blocks are
+// odd in number, 64 x 256 tiles are fewer.  They take version 13's k-loop over
+// the same sums (bitwise equal).  us per launch, fresh operands, against the
+// square tiles: 300 x 11008 x 4096 (215 for 258) 47.9 / 59.4, 192 x 16640 x 4096
+// (195 for 260) 51.1 / 60.5, 448 x 8712 x 4096 (245 for 276) 55.7 / 68.9.  A
+// 64-deep k-tile takes 0.7 us where a square tile's takes 0.46, so without a
+// round to save the square ones stay (1024 x 4096 x 4096 47.8 / 39.6).
+bool wide_grid(const GemmArgs& a) {
+  const size_t c = a.num_cus > 0 ? a.num_cus : 1;
+  const size_t square = (a.m + 127) / 128 * ((a.n + 127) / 128), wide = (a.m + 63) / 64 * ((a.n + 255) / 256);
+  return square > c && (wide + c - 1) / c < (square + c - 1) / c;
+}
+namespace pp128n {
+hipError_t launch_wide(const GemmArgs& a);
+}
+
 // Shapes on the 128 x 128 x 128 grid run without the edge treatment.
 hipError_t launch(const GemmArgs& a) {
+  if (wide_grid(a)) return pp128n::launch_wide(a);
   return a.out_dtype == VK_DTYPE_F16 ? launch_out<half_t>(a) : launch_out<float>(a);
 }
 
@@ -947,17 +965,43 @@ using pp128w::swz_a8;
 constexpr int kBK = 64;
 constexpr int kLdsBytes = kSlots * kSlot;  // 160 KB
 
-template <typename OutT, bool kEdge, bool kSplit>
+// The tile: 128 x 128, or 64 x 256 (kWide, version 11's grids with an odd
+// number of 64-row blocks, wide_grid below): every wave the same 64 x 32 block
+// of it, all 8 side by side, over a ring of 4 slots of 40 KB (A 64 rows, B 64
+// k-rows x 256 columns with version 7's swizzle), loads 3 k-tiles ahead.
+template <bool kWide>
+struct Cfg {
+  static constexpr int kTM = kWide ? 64 : kBM, kTN = kWide ? 256 : kBN;
+  static constexpr int kABytes = kTM * kARow;
+  static constexpr int kBRow = kTN * 2;
+  static constexpr int kSlot = kABytes + kBK * kBRow;
+  static constexpr int kSlots = kWide ? 4 : 5;
+  static constexpr int kAhead = kSlots - 1;            // k-tiles
+  static constexpr int kLoadsA = kTM / 64;             // per wave and k-tile, of 8 rows
+  static constexpr int kLoadsB = kTN / 64;             // of 1024 / kBRow k-rows
+  static constexpr int kLoads = kLoadsA + kLoadsB;
+  static constexpr int kRowsB = 1024 / kBRow;
+  static constexpr int kChunksB = kTN / 8;             // 16-byte chunks of a k-row
+  static_assert(kSlots * kSlot == kLdsBytes, "the whole LDS either way");
+  static __device__ constexpr int swz(int krow) {
+    return kWide ? vk::swz_b(krow) ^ (((krow >> 3) & 1) << 1) : pp128::swz_b(krow);
+  }
+};
+
+template <typename OutT, bool kEdge, bool kSplit, bool kWide = false>
 __global__ __launch_bounds__(kThreads) void f16_pp128n_kernel(const half_t* __restrict__ A,
                                                               const half_t* __restrict__ B,
                                                               OutT* __restrict__ C, int M, int N, int K, int units,
                                                               int pieces, int chunks, float* __restrict__ part,
                                                               unsigned* __restrict__ counters) {
+  using G = Cfg<kWide>;
+  constexpr int kBM = G::kTM, kBN = G::kTN, kABytes = G::kABytes, kBRow = G::kBRow, kSlot = G::kSlot;
+  constexpr int kSlots = G::kSlots, kAhead = G::kAhead, LA = G::kLoadsA, LB = G::kLoadsB, L = G::kLoads;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int grp = wave >> 2;  // rows 64 grp .. 64 grp + 63 of the tile
-  const int gw = wave & 3;    // columns 32 gw .. 32 gw + 31
+  const int grp = kWide ? 0 : wave >> 2;    // rows 64 grp .. 64 grp + 63 of the tile
+  const int gw = kWide ? wave : wave & 3;   // columns 32 gw .. 32 gw + 31
   constexpr int kR = kEdge ? 1 : 0;
   const int tiles_m = (M + kR * (kBM - 1)) / kBM, tiles_n = (N + kR * (kBN - 1)) / kBN;
   const int nk_all = (K + kR * (kBK - 1)) / kBK;
@@ -968,26 +1012,36 @@ __global__ __launch_bounds__(kThreads) void f16_pp128n_kernel(const half_t* __re
     raster_tile(w.cid, tiles_m, tiles_n, tm, tn);
     kb = 2 * w.kb;
     nk = min(2 * w.ke, nk_all) - kb;
+  } else if (kWide && tiles_m <= 8) {
+    // all tiles of a panel of B next to each other, on one XCD (300 x 11008 x
+    // 4096 47.8 us; the grouped raster 51.1, a panel's tiles spread over the
+    // XCDs 68.3)
+    const int id = xcd_remap(blockIdx.x, tiles_m * tiles_n);
+    tn = id / tiles_m;
+    tm = id - tn * tiles_m;
   } else {
     tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
   }
   const int m0 = tm * kBM, n0 = tn * kBN;
   const uint32_t lds_base = lds_addr32(lds);
 
-  // ---- loads: 4 per wave per k-tile ----
-  // A load i (0, 1): rows 16 wave + 8 i + l / 8, lane l at chunk position
-  //   l % 8, holding chunk (l % 8) ^ swz_a8(row).
-  // B load i (0, 1): k-rows 8 wave + 4 i + l / 16, position l % 16, holding
-  //   chunk (l % 16) ^ swz_b(krow).
-  uint32_t voa[2], vob[2], akin = 0;
+  // ---- loads: 4 (kWide: 5) per wave per k-tile ----
+  // A load i: rows 8 (LA wave + i) + l / 8, lane l at chunk position l % 8,
+  //   holding chunk (l % 8) ^ swz_a8(row).
+  // B load i: k-rows 8 wave + 4 i + l / 16 (kWide: 2 i + l / 32), position
+  //   l % 16 (l % 32), holding that chunk ^ swz(krow).
+  uint32_t voa[LA], vob[LB], akin = 0;
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int row = wave * 16 + 8 * i + (lane >> 3);
+  for (int i = 0; i < LA; i++) {
+    const int row = 8 * (LA * wave + i) + (lane >> 3);
     const int ca = (lane & 7) ^ swz_a8(row);
     voa[i] = (uint32_t)(((size_t)row * K + ca * 8) * 2);
     akin |= (uint32_t)(ca * 8) << (8 * i);  // kEdge: the chunk's first k within the k-tile
-    const int krow = wave * 8 + 4 * i + (lane >> 4);
-    const int cb = (lane & 15) ^ swz_b(krow);
+  }
+#pragma unroll
+  for (int i = 0; i < LB; i++) {
+    const int krow = wave * 8 + G::kRowsB * i + lane / G::kChunksB;
+    const int cb = (lane % G::kChunksB) ^ G::swz(krow);
     vob[i] = (uint32_t)(((size_t)krow * N + cb * 8) * 2);
   }
   const char* ga0 = reinterpret_cast<const char*>(A) + ((size_t)m0 * K + (size_t)kb * kBK) * 2;
@@ -1000,7 +1054,7 @@ __global__ __launch_bounds__(kThreads) void f16_pp128n_kernel(const half_t* __re
       __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(B), 0, (int)b_size, kBufferWord3);
   const uint32_t sa0 = (uint32_t)(ga0 - reinterpret_cast<const char*>(A));  // kEdge: below 2^31
   const uint32_t sb0 = (uint32_t)(gb0 - reinterpret_cast<const char*>(B));
-  const uint32_t la0 = lds_base + (uint32_t)(wave * 16 * kARow);
+  const uint32_t la0 = lds_base + (uint32_t)(wave * LA * 8 * kARow);
   const uint32_t lb0 = lds_base + (uint32_t)(kABytes + wave * 8 * kBRow);
 
   struct Ops {
@@ -1026,10 +1080,10 @@ __global__ __launch_bounds__(kThreads) void f16_pp128n_kernel(const half_t* __re
       asm volatile("" ::"s"(o.ga), "s"(o.gb));
     asm volatile("" ::"s"(o.la), "s"(o.lb));
   };
-  // load d: A for d < 2, B for d >= 2
+  // load d: A for d < LA, then B
   auto dma_with = [&](int d, const Ops& o) {
-    const int i = d & 1;
-    if (d < 2) {
+    const int i = d < LA ? d : d - LA;
+    if (d < LA) {
       if constexpr (kEdge) {
         const uint32_t off = ((akin >> (8 * i)) & 255u) < o.kleft ? voa[i] : a_size;  // a_size: zeros
         dma16_buf(ra, off, o.sa, o.la + i * 1024);
@@ -1046,7 +1100,7 @@ __global__ __launch_bounds__(kThreads) void f16_pp128n_kernel(const half_t* __re
   auto dma_all = [&](int kt, int slot) {
     const Ops o = ops_of(kt, slot);
 #pragma unroll
-    for (int d = 0; d < 4; d++) dma_with(d, o);
+    for (int d = 0; d < L; d++) dma_with(d, o);
   };
 
   // ---- fragment addresses (version 12's A rows, version 11's B columns) ----
@@ -1061,7 +1115,7 @@ __global__ __launch_bounds__(kThreads) void f16_pp128n_kernel(const half_t* __re
 #pragma unroll
   for (int j = 0; j < 2; j++) {
     const int c = gw * 4 + 2 * j + (q >> 1);
-    boff[j] = (uint32_t)(kABytes + krow0 * kBRow + 16 * (c ^ swz_b(krow0)) + 8 * (q & 1));
+    boff[j] = (uint32_t)(kABytes + krow0 * kBRow + 16 * (c ^ G::swz(krow0)) + 8 * (q & 1));
   }
 
   float4v acc[4][2];
@@ -1097,8 +1151,8 @@ __global__ __launch_bounds__(kThreads) void f16_pp128n_kernel(const half_t* __re
   };
   // One step: the 16 MFMAs of `cur` (each accumulator's 2 k-steps back to
   // back, k-step (i ^ j) & 1 first as in versions 7 and 11), after each one
-  // a read of `nxt` (when there is a next k-tile), and the 4 loads of `o`
-  // after every 4 MFMAs.
+  // a read of `nxt` (when there is a next k-tile), and the loads of `o` after
+  // every 4 MFMAs (kWide: the fifth before the last 2).
   auto step = [&](const Frags& cur, Frags& nxt, int nslot, bool has_next, const Ops& o) {
     const uint32_t sl = lds_base + (uint32_t)(nslot * kSlot);
     static_for<8>([&](auto xc) {
@@ -1113,46 +1167,46 @@ __global__ __launch_bounds__(kThreads) void f16_pp128n_kernel(const half_t* __re
       __builtin_amdgcn_sched_barrier(0);
       if (has_next) read_one(nxt, sl, std::integral_constant<int, 2 * x + 1>{});
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (x & 1) {
-        dma_with(x >> 1, o);
+      if constexpr ((x & 1) || (kWide && x == 6)) {
+        dma_with(x & 1 ? x >> 1 : 4, o);
         __builtin_amdgcn_sched_barrier(0);
       }
     });
   };
 
-  // ---- prologue: k-tiles 0..3 (a k-tile past the last one is the last one again) ----
+  // ---- prologue: the first kAhead k-tiles (one past the last is the last again) ----
 #pragma unroll
-  for (int j = 0; j < 4; j++) dma_all(min(j, nk - 1), j);
+  for (int j = 0; j < kAhead; j++) dma_all(min(j, nk - 1), j);
   Frags f0, f1;
-  wait_vmcnt<12>();  // k-tile 0
+  wait_vmcnt<(kAhead - 1) * L>();  // k-tile 0
   lds_barrier();
   read_all(f0, 0);
-  wait_vmcnt<8>();  // k-tile 1
+  wait_vmcnt<(kAhead - 2) * L>();  // k-tile 1
   lds_barrier();
   // Steps in pairs, so the two fragment sets keep their registers.
   int t = 0;
   for (; t + 1 < nk; t += 2) {
     {
-      const Ops o = ops_of(min(t + 4, nk - 1), (t + 4) % kSlots);
+      const Ops o = ops_of(min(t + kAhead, nk - 1), (t + kAhead) % kSlots);
       pin(o);
       __builtin_amdgcn_sched_barrier(0);
       step(f0, f1, (t + 1) % kSlots, true, o);
       __builtin_amdgcn_sched_barrier(0);
-      wait_vmcnt<8>();  // this wave's loads of k-tile t + 2
+      wait_vmcnt<(kAhead - 2) * L>();  // this wave's loads of k-tile t + 2
       lds_barrier();
     }
     {
-      const Ops o = ops_of(min(t + 5, nk - 1), (t + 5) % kSlots);
+      const Ops o = ops_of(min(t + 1 + kAhead, nk - 1), (t + 1 + kAhead) % kSlots);
       pin(o);
       __builtin_amdgcn_sched_barrier(0);
       step(f1, f0, (t + 2) % kSlots, t + 2 < nk, o);
       __builtin_amdgcn_sched_barrier(0);
-      wait_vmcnt<8>();  // this wave's loads of k-tile t + 3
+      wait_vmcnt<(kAhead - 2) * L>();  // this wave's loads of k-tile t + 3
       lds_barrier();
     }
   }
   if (t < nk) {  // an odd last k-tile
-    const Ops o = ops_of(nk - 1, (t + 4) % kSlots);
+    const Ops o = ops_of(nk - 1, (t + kAhead) % kSlots);
     pin(o);
     __builtin_amdgcn_sched_barrier(0);
     step(f0, f1, 0, false, o);
@@ -1211,6 +1265,27 @@ hipError_t launch_t(const GemmArgs& a, const SkPlan& p) {
                      static_cast<const half_t*>(a.A), static_cast<const half_t*>(a.B), static_cast<OutT*>(a.C),
                      (int)a.m, (int)a.n, (int)a.k, p.units, p.pieces, p.chunks, part, counters);
   return hipGetLastError();
+}
+
+// 64 x 256 tiles, whole.
+template <typename OutT, bool kEdge>
+hipError_t launch_wide_t(const GemmArgs& a) {
+  static std::atomic<uint64_t> attr_done{0};
+  auto kfn = f16_pp128n_kernel<OutT, kEdge, false, true>;
+  hipError_t e = ensure_lds_attr(kfn, kLdsBytes, a.device, attr_done);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kfn, dim3((unsigned)(((a.m + 63) / 64) * ((a.n + 255) / 256))), dim3(kThreads), kLdsBytes,
+                     a.stream, static_cast<const half_t*>(a.A), static_cast<const half_t*>(a.B),
+                     static_cast<OutT*>(a.C), (int)a.m, (int)a.n, (int)a.k, 0, 1, 1, nullptr, nullptr);
+  return hipGetLastError();
+}
+template <typename OutT>
+hipError_t launch_wide_out(const GemmArgs& a) {
+  const bool grid = a.m % 64 == 0 && a.n % 256 == 0 && a.k % kBK == 0;
+  return grid ? launch_wide_t<OutT, false>(a) : launch_wide_t<OutT, true>(a);
+}
+hipError_t launch_wide(const GemmArgs& a) {
+  return a.out_dtype == VK_DTYPE_F16 ? launch_wide_out<half_t>(a) : launch_wide_out<float>(a);
 }
 
 template <typename OutT>
