@@ -118,7 +118,7 @@ bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
 }
 
 hipError_t launch_padded(const GemmArgs& a) {
-  if (few_rows(a.m, a.n, a.k)) return f16_stream_launch(a);
+  if (few_rows(a.m, a.n, a.k)) return f16_stream_launch(a, layout_of(a.m, a.n, a.k, a.num_cus).total);
   if (no_copies(a.m, a.n, a.k, a.num_cus)) return f16_any_launch(a);
   const KernelEntry* inner = find_registered(kInnerVersion, VK_DTYPE_F16);
   if (!inner) return hipErrorInvalidValue;
@@ -152,8 +152,7 @@ hipError_t launch_padded(const GemmArgs& a) {
 // fp32 C of n8 columns, also those that use less of it or none, so the sizes
 // that callers hold workspaces for stay what they have been.
 size_t workspace_padded(size_t m, size_t n, size_t k, int num_cus) {
-  const size_t total = layout_of(m, n, k, num_cus).total;
-  return few_rows(m, n, k) ? std::max(total, f16_stream_workspace(m, n, k, num_cus)) : total;
+  return layout_of(m, n, k, num_cus).total;
 }
 
 // Calls of few rows leave their own counters clean at the workspace's start,

@@ -216,13 +216,10 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
 int halves_of(size_t m) { return m > 64 ? 2 : 1; }
 int blocks_of(size_t m) { return (int)(((m + 15) / 16 + halves_of(m) - 1) / halves_of(m)); }
 
-int pieces_of(size_t m, size_t n, size_t k, int num_cus) {
-  return stream_pieces((n + kNC - 1) / kNC * halves_of(m), k / kKStep, num_cus);
-}
-
 template <int MB, typename OutT>
-hipError_t launch_t(const GemmArgs& a) {
-  const int ks = pieces_of(a.m, a.n, a.k, a.num_cus), halves = halves_of(a.m);
+hipError_t launch_t(const GemmArgs& a, size_t ws_limit) {
+  const int halves = halves_of(a.m);
+  const int ks = stream_pieces((a.n + kNC - 1) / kNC * halves, a.k / kKStep, MB, 2, ws_limit, a.num_cus);
   unsigned* counters = nullptr;
   float* part = nullptr;
   const hipError_t e = stream_buffers(a, ks, counters, part);
@@ -235,8 +232,8 @@ hipError_t launch_t(const GemmArgs& a) {
 }
 
 template <int MB>
-hipError_t launch_mb(const GemmArgs& a) {
-  return a.out_dtype == VK_DTYPE_F16 ? launch_t<MB, half_t>(a) : launch_t<MB, float>(a);
+hipError_t launch_mb(const GemmArgs& a, size_t ws_limit) {
+  return a.out_dtype == VK_DTYPE_F16 ? launch_t<MB, half_t>(a, ws_limit) : launch_t<MB, float>(a, ws_limit);
 }
 
 }  // namespace
@@ -247,17 +244,12 @@ bool f16_stream_takes(size_t m, size_t n, size_t k) {
   return m >= 1 && m <= kMaxRows && n >= 8 && n < (1u << 25) && k >= 8 * W * kKStep && k < (1u << 23);
 }
 
-size_t f16_stream_workspace(size_t m, size_t n, size_t k, int num_cus) {
-  const int ks = pieces_of(m, n, k, num_cus);
-  return stream_workspace((n + kNC - 1) / kNC * halves_of(m), ks, blocks_of(m), 2);
-}
-
-hipError_t f16_stream_launch(const GemmArgs& a) {
+hipError_t f16_stream_launch(const GemmArgs& a, size_t ws_limit) {
   switch (blocks_of(a.m)) {
-    case 1: return launch_mb<1>(a);
-    case 2: return launch_mb<2>(a);
-    case 3: return launch_mb<3>(a);
-    default: return launch_mb<4>(a);
+    case 1: return launch_mb<1>(a, ws_limit);
+    case 2: return launch_mb<2>(a, ws_limit);
+    case 3: return launch_mb<3>(a, ws_limit);
+    default: return launch_mb<4>(a, ws_limit);
   }
 }
 

@@ -851,8 +851,7 @@ hipError_t launch_f32_small(const GemmArgs& a) {
   return f32_small_nb(a.m, a.n, a.num_cus) == 1 ? launch_f32_small_nb<1, kEdge>(a) : launch_f32_small_nb<2, kEdge>(a);
 }
 
-// Workspace of versions 2 and 3 (but few rows): the split's counters and
-// partials.
+// Workspace of versions 2 and 3: the split's counters and partials.
 size_t f32_workspace(size_t m, size_t n, size_t k, int num_cus) {
   if (!f32_small_tiles(m, n, num_cus) || (k % 32 != 0 && !f32_mfma_edge_shape_ok(m, n, k))) return 0;
   const int nb = f32_small_nb(m, n, num_cus);
@@ -895,9 +894,9 @@ bool f32_mfma_shape_ok(size_t m, size_t n, size_t k) {
 // Version 3 (any M; N, K multiples of 4): 32-deep k-tiles (the last one
 // masked where K % 32 != 0); each operand below 2^31 bytes (buffer sizes and
 // offsets).
-// Few rows: f32_stream.hip.
+// Few rows: f32_stream.hip, within the workspace of the tiles' split.
 hipError_t launch_f32_mfma_edge(const GemmArgs& a) {
-  if (f32_stream_takes(a.m, a.n, a.k)) return f32_stream_launch(a);
+  if (f32_stream_takes(a.m, a.n, a.k)) return f32_stream_launch(a, f32_workspace(a.m, a.n, a.k, a.num_cus));
   if (f32_small_tiles(a.m, a.n, a.num_cus)) return launch_f32_small<true>(a);
   return a.k % 32 == 0 ? launch_w4<4, true, false>(a, SkPlan{0, 0, 1, 1}) : launch_bk<32, true>(a);
 }
@@ -905,10 +904,6 @@ hipError_t launch_f32_mfma_edge(const GemmArgs& a) {
 bool f32_mfma_edge_shape_ok(size_t m, size_t n, size_t k) {
   return m >= 1 && n >= 4 && k >= 4 && m * k * 4 < (1ull << 31) && k * n * 4 < (1ull << 31) &&
          f32_mfma_shape_ok(((m + kBM - 1) / kBM) * kBM, ((n + kBN - 1) / kBN) * kBN, k);
-}
-
-size_t f32_workspace_edge(size_t m, size_t n, size_t k, int num_cus) {
-  return f32_stream_takes(m, n, k) ? f32_stream_workspace(m, n, k, num_cus) : f32_workspace(m, n, k, num_cus);
 }
 
 }  // namespace
@@ -931,7 +926,6 @@ void register_f32_mfma() {
   e3.caps = make_caps(3, VK_DTYPE_F32, kOutF32, 1, 4, 4, 16, kBM, kBN, 32, 256, F32Cfg<32>::kLdsBytes, 0, 0);
   e3.caps.uses_workspace = 1;
   e3.launch = launch_f32_mfma_edge;
-  e3.workspace = f32_workspace_edge;
   e3.shape_ok = f32_mfma_edge_shape_ok;
   register_kernel(e3);
 }

@@ -150,14 +150,11 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f32_stream_kernel(c
                        });
 }
 
-int pieces_of(size_t n, size_t k, int num_cus) {
-  return stream_pieces((n + kNC - 1) / kNC, (k + kKStep - 1) / kKStep, num_cus);
-}
 int blocks_of(size_t m) { return (int)((m + 15) / 16); }
 
 template <int MB>
-hipError_t launch_mb(const GemmArgs& a) {
-  const int ks = pieces_of(a.n, a.k, a.num_cus);
+hipError_t launch_mb(const GemmArgs& a, size_t ws_limit) {
+  const int ks = stream_pieces((a.n + kNC - 1) / kNC, (a.k + kKStep - 1) / kKStep, MB, 1, ws_limit, a.num_cus);
   unsigned* counters = nullptr;
   float* part = nullptr;
   const hipError_t e = stream_buffers(a, ks, counters, part);
@@ -185,16 +182,12 @@ bool f32_stream_takes(size_t m, size_t n, size_t k) {
   return m >= 1 && m <= kMaxRows && n >= 4 && n % 4 == 0 && n < (1u << 25) && k >= 4 && k % 4 == 0 && k < (1u << 23);
 }
 
-size_t f32_stream_workspace(size_t m, size_t n, size_t k, int num_cus) {
-  return stream_workspace((n + kNC - 1) / kNC, pieces_of(n, k, num_cus), blocks_of(m), 1);
-}
-
-hipError_t f32_stream_launch(const GemmArgs& a) {
+hipError_t f32_stream_launch(const GemmArgs& a, size_t ws_limit) {
   switch (blocks_of(a.m)) {
-    case 1: return launch_mb<1>(a);
-    case 2: return launch_mb<2>(a);
-    case 3: return launch_mb<3>(a);
-    default: return launch_mb<4>(a);
+    case 1: return launch_mb<1>(a, ws_limit);
+    case 2: return launch_mb<2>(a, ws_limit);
+    case 3: return launch_mb<3>(a, ws_limit);
+    default: return launch_mb<4>(a, ws_limit);
   }
 }
 

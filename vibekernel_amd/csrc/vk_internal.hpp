@@ -61,18 +61,17 @@ const KernelEntry* find_registered(int version, vk_dtype in);
 // fp32, any shape and alignment (f32_any.hip).
 hipError_t f32_any_launch(const GemmArgs& a);
 
-// fp32, few rows, N and K multiples of 4 (f32_stream.hip).
+// fp32, few rows, N and K multiples of 4 (f32_stream.hip), with at most
+// ws_limit bytes of the workspace.
 bool f32_stream_takes(size_t m, size_t n, size_t k);
-size_t f32_stream_workspace(size_t m, size_t n, size_t k, int num_cus);
-hipError_t f32_stream_launch(const GemmArgs& a);
+hipError_t f32_stream_launch(const GemmArgs& a, size_t ws_limit);
 
 // fp16, any shape and alignment (f16_any.hip).
 hipError_t f16_any_launch(const GemmArgs& a);
 
-// fp16, few rows, any N >= 8 and K (f16_stream.hip).
+// fp16, few rows, N >= 8 and K >= 1024 (f16_stream.hip), the same.
 bool f16_stream_takes(size_t m, size_t n, size_t k);
-size_t f16_stream_workspace(size_t m, size_t n, size_t k, int num_cus);
-hipError_t f16_stream_launch(const GemmArgs& a);
+hipError_t f16_stream_launch(const GemmArgs& a, size_t ws_limit);
 
 // Fill `words` 32-bit words with zero on `stream` (a kernel, not
 // hipMemsetAsync, so it may be captured into a graph).

@@ -8,8 +8,6 @@
 // workgroups of a column block.
 #pragma once
 
-#include <algorithm>
-
 #include "vk_device.hpp"
 #include "vk_internal.hpp"
 
@@ -24,17 +22,16 @@ constexpr size_t kStreamCounterBytes = 8192;  // a counter per (block, wave)
 // fp32 27.0 us instead of 24.1, 16 x 4095 x 4096 fp16 25.9 instead of 16.8.)
 // The pieces of a block belong on different XCDs: dealt next to each other
 // these two took 24.1 and 16.8 us, spread 19.1 and 13.7.
-inline int stream_pieces(size_t blocks, size_t steps, int num_cus) {
+// The counters and a slot of 4 waves x mb h KB per piece (mb row blocks, h
+// groups of 4 columns per lane) stay within ws_limit bytes.
+inline int stream_pieces(size_t blocks, size_t steps, int mb, int h, size_t ws_limit, int num_cus) {
+  const size_t slot = (size_t)kStreamWaves * mb * h * 1024;
   int ks = 1;
   if (blocks * kStreamWaves * sizeof(unsigned) > kStreamCounterBytes) return 1;
-  while (ks < kStreamMaxPieces && blocks * ks * 2 <= (size_t)num_cus && steps / (ks * 2) >= 4 * kStreamWaves) ks *= 2;
+  while (ks < kStreamMaxPieces && blocks * ks * 2 <= (size_t)num_cus && steps / (ks * 2) >= 4 * kStreamWaves &&
+         kStreamCounterBytes + blocks * ks * 2 * slot <= ws_limit)
+    ks *= 2;
   return ks;
-}
-
-// Counters (the same place for every shape), then a slot of 4 waves x MB H KB
-// per piece.
-inline size_t stream_workspace(size_t blocks, int ks, int mb, int h) {
-  return ks == 1 ? 0 : kStreamCounterBytes + blocks * ks * kStreamWaves * (size_t)mb * h * 1024;
 }
 
 inline hipError_t stream_buffers(const GemmArgs& a, int ks, unsigned*& counters, float*& part) {
