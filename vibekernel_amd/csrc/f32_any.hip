@@ -237,8 +237,9 @@ hipError_t launch_any(const GemmArgs& a) {
 hipError_t f32_any_launch(const GemmArgs& a) {
   const size_t c = a.num_cus > 0 ? a.num_cus : 1;
   const size_t big = (a.m + 127) / 128 * ((a.n + 127) / 128), small = (a.m + 63) / 64 * ((a.n + 63) / 64);
-  // grid.y holds up to 65535 rows of tiles
-  const bool use_small = 4 * ((big + c - 1) / c) > (small + c - 1) / c && (a.m + 63) / 64 <= 65535;
+  // grid.y holds up to 65535 rows of tiles, grid.x up to 2^32 - 1 threads
+  const bool use_small = 4 * ((big + c - 1) / c) > (small + c - 1) / c && (a.m + 63) / 64 <= 65535 &&
+                         (a.n + 63) / 64 < ((size_t)1 << 32) / kThreads;
   return use_small ? launch_any<1>(a) : launch_any<2>(a);
 }
 

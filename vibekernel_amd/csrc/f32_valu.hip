@@ -31,9 +31,6 @@ constexpr int kCG = 4;               // 64-column groups per tile
 constexpr int kTN = 64 * kCG;        // tile columns
 constexpr int kBK = 16;
 constexpr int kApitch = kTM + 4;     // As_t[k][m] row pitch (floats)
-constexpr int kLdA = kTM * kBK / 4 / 256;  // float4 loads of A per thread per k-tile
-constexpr int kLdB = kBK * kTN / 4 / 256;  // float4 loads of B per thread per k-tile
-static_assert(kLdA == 2 && kLdB == 4, "tile load mapping");
 
 // Every VGPR from v32 up: the registers the asm kernel below uses itself.
 #define VK_CLOBBER_V32_V255 \
