@@ -63,9 +63,10 @@ def test_values_past_the_edges_and_guards(gpu, shape):
 
 
 def test_repeats_and_shared_workspace(gpu):
-    """A split shape between calls whose workspace holds copies there."""
+    """A split shape between calls whose workspace holds copies there (past
+    2^33 multiply-adds, 256 whole tiles: the copy of B is at its start)."""
     A, B = make_inputs(33, 1001, 4097, "normal", seed=3)
-    A2, B2 = make_inputs(300, 1001, 1000, "normal", seed=4)
+    A2, B2 = make_inputs(4096, 4095, 1032, "normal", seed=4)
     ref, ref2 = run_gemm(15, A, B, "f32"), run_gemm(15, A2, B2, "f32")
     for _ in range(3):
         assert np.array_equal(run_gemm(15, A, B, "f32"), ref)

@@ -155,9 +155,14 @@ size_t workspace_padded(size_t m, size_t n, size_t k, int num_cus) {
   return layout_of(m, n, k, num_cus).total;
 }
 
-// Calls of few rows leave their own counters clean at the workspace's start,
-// the others do not.
-int workspace_kind(size_t m, size_t n, size_t k) { return few_rows(m, n, k) ? 1 : 0; }
+// Calls of few rows that split K leave their own counters clean at the
+// workspace's start; those that do not, and calls without copies, leave it as
+// it was, whatever it holds; the copies overwrite it.
+int workspace_kind(size_t m, size_t n, size_t k, int num_cus) {
+  if (few_rows(m, n, k))
+    return f16_stream_pieces(m, n, k, layout_of(m, n, k, num_cus).total, num_cus) > 1 ? 1 : kWorkspaceUntouched;
+  return no_copies(m, n, k, num_cus) ? kWorkspaceUntouched : 0;
+}
 
 // Version 10's limits on the padded problem.
 bool shape_ok_padded(size_t m, size_t n, size_t k) {

@@ -219,7 +219,7 @@ int blocks_of(size_t m) { return (int)(((m + 15) / 16 + halves_of(m) - 1) / halv
 template <int MB, typename OutT>
 hipError_t launch_t(const GemmArgs& a, size_t ws_limit) {
   const int halves = halves_of(a.m);
-  const int ks = stream_pieces((a.n + kNC - 1) / kNC * halves, a.k / kKStep, MB, 2, ws_limit, a.num_cus);
+  const int ks = f16_stream_pieces(a.m, a.n, a.k, ws_limit, a.num_cus);
   unsigned* counters = nullptr;
   float* part = nullptr;
   const hipError_t e = stream_buffers(a, ks, counters, part);
@@ -242,6 +242,10 @@ hipError_t launch_mb(const GemmArgs& a, size_t ws_limit) {
 // 32 k-rows of B and 128 rows of A below 2^32 bytes.
 bool f16_stream_takes(size_t m, size_t n, size_t k) {
   return m >= 1 && m <= kMaxRows && n >= 8 && n < (1u << 25) && k >= 8 * W * kKStep && k < (1u << 23);
+}
+
+int f16_stream_pieces(size_t m, size_t n, size_t k, size_t ws_limit, int num_cus) {
+  return stream_pieces((n + kNC - 1) / kNC * halves_of(m), k / kKStep, blocks_of(m), 2, ws_limit, num_cus);
 }
 
 hipError_t f16_stream_launch(const GemmArgs& a, size_t ws_limit) {

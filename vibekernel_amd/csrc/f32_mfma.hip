@@ -901,6 +901,14 @@ hipError_t launch_f32_mfma_edge(const GemmArgs& a) {
   return a.k % 32 == 0 ? launch_w4<4, true, false>(a, SkPlan{0, 0, 1, 1}) : launch_bk<32, true>(a);
 }
 
+// Few rows and tiles keep their counters in the same place and leave them at
+// zero; few rows whose K is not split leave the workspace as it was.
+int f32_edge_workspace_kind(size_t m, size_t n, size_t k, int num_cus) {
+  const bool unsplit =
+      f32_stream_takes(m, n, k) && f32_stream_pieces(m, n, k, f32_workspace(m, n, k, num_cus), num_cus) == 1;
+  return unsplit ? kWorkspaceUntouched : 0;
+}
+
 bool f32_mfma_edge_shape_ok(size_t m, size_t n, size_t k) {
   return m >= 1 && n >= 4 && k >= 4 && m * k * 4 < (1ull << 31) && k * n * 4 < (1ull << 31) &&
          f32_mfma_shape_ok(((m + kBM - 1) / kBM) * kBM, ((n + kBN - 1) / kBN) * kBN, k);
@@ -927,6 +935,7 @@ void register_f32_mfma() {
   e3.caps.uses_workspace = 1;
   e3.launch = launch_f32_mfma_edge;
   e3.shape_ok = f32_mfma_edge_shape_ok;
+  e3.workspace_kind = f32_edge_workspace_kind;
   register_kernel(e3);
 }
 

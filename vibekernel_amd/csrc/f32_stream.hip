@@ -154,7 +154,7 @@ int blocks_of(size_t m) { return (int)((m + 15) / 16); }
 
 template <int MB>
 hipError_t launch_mb(const GemmArgs& a, size_t ws_limit) {
-  const int ks = stream_pieces((a.n + kNC - 1) / kNC, (a.k + kKStep - 1) / kKStep, MB, 1, ws_limit, a.num_cus);
+  const int ks = f32_stream_pieces(a.m, a.n, a.k, ws_limit, a.num_cus);
   unsigned* counters = nullptr;
   float* part = nullptr;
   const hipError_t e = stream_buffers(a, ks, counters, part);
@@ -180,6 +180,10 @@ hipError_t launch_mb(const GemmArgs& a, size_t ws_limit) {
 bool f32_stream_takes(size_t m, size_t n, size_t k) {
   if (m > 32 && n * k < ((size_t)1 << 23)) return false;
   return m >= 1 && m <= kMaxRows && n >= 4 && n % 4 == 0 && n < (1u << 25) && k >= 4 && k % 4 == 0 && k < (1u << 23);
+}
+
+int f32_stream_pieces(size_t m, size_t n, size_t k, size_t ws_limit, int num_cus) {
+  return stream_pieces((n + kNC - 1) / kNC, (k + kKStep - 1) / kKStep, blocks_of(m), 1, ws_limit, num_cus);
 }
 
 hipError_t f32_stream_launch(const GemmArgs& a, size_t ws_limit) {

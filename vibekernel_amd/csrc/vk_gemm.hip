@@ -197,9 +197,9 @@ int run(int version, vk_dtype in, vk_dtype out, size_t m, size_t n, size_t k, co
   if (device_state(dev, &ds) != hipSuccess) return VK_ERR_HIP;
 
   const size_t need = e->workspace ? e->workspace(m, n, k, ds->num_cus) : 0;
-  const int kind = e->workspace_kind ? e->workspace_kind(m, n, k) : 0;
   bool ws_clean = false;
-  bool owns_ws = false;  // this call uses the library workspace
+  int kind = 0;
+  bool owns_ws = false;  // this call reads or writes the library workspace
   if (need > 0) {
     if (library_ws) {
       // A graph captured now would keep this workspace's address, which a
@@ -222,12 +222,15 @@ int run(int version, vk_dtype in, vk_dtype out, size_t m, size_t n, size_t k, co
       }
       ws = ds->ws;
       ws_bytes = ds->ws_bytes;
-      ws_clean = ds->ws_entry == e && ds->ws_kind == kind;
-      // Until this launch is known to have been enqueued, the counters count
-      // as unknown: a failed launch must not leave the next call skipping the
-      // clear.
-      ds->ws_entry = nullptr;
-      owns_ws = true;
+      kind = e->workspace_kind ? e->workspace_kind(m, n, k, ds->num_cus) : 0;
+      if (kind != kWorkspaceUntouched) {
+        ws_clean = ds->ws_entry == e && ds->ws_kind == kind;
+        // Until this launch is known to have been enqueued, the counters count
+        // as unknown: a failed launch must not leave the next call skipping the
+        // clear.
+        ds->ws_entry = nullptr;
+        owns_ws = true;
+      }
     } else if (!ws || ws_bytes < need) {
       return VK_ERR_WORKSPACE;
     }

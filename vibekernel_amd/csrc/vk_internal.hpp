@@ -38,8 +38,12 @@ using LaunchFn = hipError_t (*)(const GemmArgs&);
 using WorkspaceFn = size_t (*)(size_t m, size_t n, size_t k, int num_cus);
 // Optional extra shape rule beyond the divisibility in caps (nullptr = none).
 using ShapeFn = bool (*)(size_t m, size_t n, size_t k);
-// Which of a version's workspace layouts a shape takes (nullptr: it has one).
-using KindFn = int (*)(size_t m, size_t n, size_t k);
+// Which of a version's workspace layouts a shape's launch takes (nullptr: it has
+// one), or kWorkspaceUntouched where it asks for a workspace (its size is part
+// of the interface) and then neither reads nor writes it: such a call says
+// nothing about the counters there.
+using KindFn = int (*)(size_t m, size_t n, size_t k, int num_cus);
+constexpr int kWorkspaceUntouched = -1;
 
 struct KernelEntry {
   int version;
@@ -62,8 +66,10 @@ const KernelEntry* find_registered(int version, vk_dtype in);
 hipError_t f32_any_launch(const GemmArgs& a);
 
 // fp32, few rows, N and K multiples of 4 (f32_stream.hip), with at most
-// ws_limit bytes of the workspace.
+// ws_limit bytes of the workspace: none where _pieces, the workgroups per
+// column block, is 1.
 bool f32_stream_takes(size_t m, size_t n, size_t k);
+int f32_stream_pieces(size_t m, size_t n, size_t k, size_t ws_limit, int num_cus);
 hipError_t f32_stream_launch(const GemmArgs& a, size_t ws_limit);
 
 // fp16, any shape and alignment (f16_any.hip).
@@ -71,6 +77,7 @@ hipError_t f16_any_launch(const GemmArgs& a);
 
 // fp16, few rows, N >= 8 and K >= 1024 (f16_stream.hip), the same.
 bool f16_stream_takes(size_t m, size_t n, size_t k);
+int f16_stream_pieces(size_t m, size_t n, size_t k, size_t ws_limit, int num_cus);
 hipError_t f16_stream_launch(const GemmArgs& a, size_t ws_limit);
 
 // Fill `words` 32-bit words with zero on `stream` (a kernel, not

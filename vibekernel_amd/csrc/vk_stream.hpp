@@ -34,6 +34,9 @@ inline int stream_pieces(size_t blocks, size_t steps, int mb, int h, size_t ws_l
   return ks;
 }
 
+// The workspace of ks pieces: the counters, cleared unless they are known to be
+// zero, then the partial slots.  One piece touches nothing there
+// (kWorkspaceUntouched), so its call is no word on the counters either.
 inline hipError_t stream_buffers(const GemmArgs& a, int ks, unsigned*& counters, float*& part) {
   if (ks == 1) return hipSuccess;
   counters = static_cast<unsigned*>(a.workspace);
