@@ -1,53 +1,18 @@
 """The library workspace's counters on the host: libvk_gemm.so's own launch code
-over a stand-in HIP runtime (tests/native/hip_stub.cpp) that logs launches.
-Fresh and reused memory holds garbage there, so a launch that counts arrivals
-must find its counters at zero, whatever calls came before it and whether they
-split K, copied operands to the workspace's start or left it alone.  The GPU
-counterpart is tests/test_gpu_workspace_counters.py."""
-import json
-import os
-import subprocess
-import sys
-
+over a stand-in HIP runtime that logs launches (host_launches.py).  Fresh and
+reused memory holds garbage there, so a launch that counts arrivals must find
+its counters at zero, whatever calls came before it and whether they split K,
+copied operands to the workspace's start or left it alone.  The GPU counterpart
+is tests/test_gpu_workspace_counters.py."""
 import pytest
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-STUB = os.path.join(ROOT, "tests", "native", "hip_stub.cpp")
-LIB = os.path.join(ROOT, "vibekernel_amd", "lib", "libvk_gemm.so")
-
-# In a process of its own: the stand-in has to be there before any HIP runtime.
-CHILD = """
-import ctypes, json, sys
-stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-stub.stub_log.restype = ctypes.c_char_p
-lib = ctypes.CDLL(sys.argv[2])
-lib.vk_gemm.argtypes = [ctypes.c_int] * 3 + [ctypes.c_size_t] * 3 + [ctypes.c_void_p] * 4
-done, out = 0, []
-for dtype, version, m, n, k in json.loads(sys.argv[3]):
-    status = lib.vk_gemm(version, dtype, dtype, m, n, k, 4096, 4096, 4096, None)
-    lines = stub.stub_log().decode().splitlines()
-    out.append([status, lines[done:]])
-    done = len(lines)
-print(json.dumps(out))
-"""
+import host_launches
 
 
 @pytest.fixture(scope="module")
 def launches(tmp_path_factory):
-    """[(status, launch lines)] of a list of calls (dtype 1: fp16, 2: fp32) in a
-    fresh process."""
-    if not os.path.exists(LIB):
-        pytest.fail(f"{LIB} is not built")
-    stub = str(tmp_path_factory.mktemp("stub") / "libhip_stub.so")
-    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", STUB, "-o", stub], check=True, timeout=300)
-
-    def run(calls):
-        r = subprocess.run([sys.executable, "-c", CHILD, stub, LIB, json.dumps(calls)], capture_output=True, text=True,
-                           timeout=300)
-        assert r.returncode == 0, r.stdout + r.stderr
-        return json.loads(r.stdout.splitlines()[-1])
-
-    return run
+    stub = host_launches.build_stub(tmp_path_factory.mktemp("stub"))
+    return lambda calls: host_launches.launches(stub, calls)
 
 
 def v15(*shape):

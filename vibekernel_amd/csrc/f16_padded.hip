@@ -114,6 +114,7 @@ bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_str
 // tiles of a deep K keep version 10's split sum (300 x 200 x 4095: 28.7 / 49).
 bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
   const size_t tiles = (m + 63) / 64 * ((n + 63) / 64);
+  if ((m + 127) / 128 > 65535) return false;  // rows of its tiles are grid.y
   return (n % 8 || k % 8) && m * n * k <= ((size_t)1 << 33) && (8 * tiles >= (size_t)num_cus || k <= 1024);
 }
 
