@@ -25,3 +25,20 @@ def test_tall_f16(gpu):
     vk.matmul(m, n, k, A.half(), B.half(), C, version)
     torch.cuda.synchronize()
     assert torch.equal(C, exact.half())
+
+
+def test_wide_f32(gpu):
+    """One row of 2^30 + 77 columns: more than 2^32 threads in one row of
+    tiles."""
+    import torch
+    import vibekernel_amd as vk
+    n = 2 ** 30 + 77
+    A = torch.tensor([[3.0]], device="cuda:0")
+    B = (torch.arange(n, device="cuda:0", dtype=torch.int32) % 1000003).float().view(1, n)
+    C = torch.full((1, n), float("nan"), device="cuda:0")
+    version = vk.pick_version(1, n, 1, "f32")
+    announce(f"wide f32 version={version} n={n}")
+    assert version == 1
+    vk.matmul(1, n, 1, A, B, C, version)
+    torch.cuda.synchronize()
+    assert torch.equal(C, 3 * B)

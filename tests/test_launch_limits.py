@@ -20,7 +20,8 @@ def launches(tmp_path_factory):
 
 # (dtype, version, m, n, k), all accepted by vk_gemm_check
 SHAPES = [(F16, 15, 9000000, 9, 8), (F16, 15, 65535 * 128 + 1, 1, 100), (F16, 15, 65535 * 128, 9, 8),
-          (F16, 1, 65535 * 128, 9, 8), (F32, 1, 65535 * 128, 3, 5)]
+          (F16, 1, 65535 * 128, 9, 8), (F32, 1, 65535 * 128, 3, 5),
+          (F32, 1, 65, 2 ** 30, 1), (F32, 1, 1, 2 ** 30 + 77, 1), (F32, 1, 70, 2 ** 29 + 5, 2)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)

@@ -36,6 +36,8 @@
 #include "vk_internal.hpp"
 #include "vk_tile.hpp"
 
+#include <algorithm>
+
 namespace vk {
 namespace {
 
@@ -67,8 +69,10 @@ __global__ __launch_bounds__(kThreads, NB == 1 ? 4 : 2) void f32_any_kernel(cons
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, l16 = lane & 15;
+  const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+  if (id >= tiles_m * tiles_n) return;  // the last row of a folded grid
   int tm, tn;
-  tile_of((int)(blockIdx.y * gridDim.x + blockIdx.x), tiles_m, tiles_n, tm, tn);
+  tile_of(id, tiles_m, tiles_n, tm, tn);
   const int64_t m0 = (int64_t)tm * T, n0 = (int64_t)tn * T;
 
   // Chunk i of this thread: 4 k of a row of A, 4 columns of a k-row of B.
@@ -224,7 +228,10 @@ __global__ __launch_bounds__(kThreads, NB == 1 ? 4 : 2) void f32_any_kernel(cons
 template <int NB>
 hipError_t launch_any(const GemmArgs& a) {
   const size_t tm = (a.m + AnyCfg<NB>::kT - 1) / AnyCfg<NB>::kT, tn = (a.n + AnyCfg<NB>::kT - 1) / AnyCfg<NB>::kT;
-  hipLaunchKernelGGL(f32_any_kernel<NB>, dim3((unsigned)tn, (unsigned)tm), dim3(kThreads), 0, a.stream,
+  // A row of tiles per grid.y, or, where that is too wide, the tiles in rows as
+  // wide as a grid may be (fewer than 2^32 threads).
+  const size_t gx = std::min(tn, (((size_t)1 << 32) - 1) / kThreads), gy = gx == tn ? tm : (tm * tn + gx - 1) / gx;
+  hipLaunchKernelGGL(f32_any_kernel<NB>, dim3((unsigned)gx, (unsigned)gy), dim3(kThreads), 0, a.stream,
                      static_cast<const float*>(a.A), static_cast<const float*>(a.B), static_cast<float*>(a.C),
                      (int64_t)a.m, (int64_t)a.n, (int64_t)a.k, (int)tm, (int)tn);
   return hipGetLastError();
@@ -237,9 +244,8 @@ hipError_t launch_any(const GemmArgs& a) {
 hipError_t f32_any_launch(const GemmArgs& a) {
   const size_t c = a.num_cus > 0 ? a.num_cus : 1;
   const size_t big = (a.m + 127) / 128 * ((a.n + 127) / 128), small = (a.m + 63) / 64 * ((a.n + 63) / 64);
-  // grid.y holds up to 65535 rows of tiles, grid.x up to 2^32 - 1 threads
-  const bool use_small = 4 * ((big + c - 1) / c) > (small + c - 1) / c && (a.m + 63) / 64 <= 65535 &&
-                         (a.n + 63) / 64 < ((size_t)1 << 32) / kThreads;
+  // grid.y holds up to 65535 rows of tiles
+  const bool use_small = 4 * ((big + c - 1) / c) > (small + c - 1) / c && (a.m + 63) / 64 <= 65535;
   return use_small ? launch_any<1>(a) : launch_any<2>(a);
 }
 
