@@ -1,0 +1,34 @@
+"""Which kernel a call launches, on the host: libvk_gemm.so's own launch code
+over a stand-in HIP runtime that logs launches (host_launches.py; 256 CUs).
+Each case lies on one side of a rule whose two sides are measured where it
+stands in the source."""
+import pytest
+
+import host_launches
+
+F16, F32 = 1, 2
+
+
+@pytest.fixture(scope="module")
+def kernel(tmp_path_factory):
+    """The (mangled) name of the last kernel that one call launches."""
+    stub = host_launches.build_stub(tmp_path_factory.mktemp("stub"))
+
+    def run(*call):
+        (status, lines), = host_launches.launches(stub, [list(call)])
+        assert status == 0, call
+        return lines[-1].split()[0]
+
+    return run
+
+
+# C's rows on 16-byte boundaries or not: the last template argument
+@pytest.mark.parametrize("call,name", [
+    ((F16, 10, 520, 520, 64), "f16_pp16_edge_kernelIDF16_Lb0EE"),
+    ((F16, 10, 1000, 1000, 4000), "f16_pp16_sk_kernelIDF16_Lb1ELb0EE"),
+    ((F16, 15, 4096, 4096, 4095), "f16_pp16_edge_kernelIDF16_Lb0EE"),
+    ((F16, 15, 4096, 4095, 4096), "f16_pp16_edge_kernelIDF16_Lb1EE"),
+    ((F16, 15, 300, 201, 4095), "f16_pp16_sk_kernelIDF16_Lb1ELb1EE"),
+])
+def test_rows_of_c_in_version_10(kernel, call, name):
+    assert name in kernel(*call)

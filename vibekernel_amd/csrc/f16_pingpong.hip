@@ -612,12 +612,16 @@ static_assert(lds_bytes_of<kAblB2>() >= 8 * 128 * 64 * 2, "fp16 epilogue staging
 template <typename OutT>
 struct Epi16;
 
-// 16 bytes of a row of C that has `left` elements from there on.
+// 16 bytes of a row of C that has `left` elements from there on.  kAny: rows of
+// any length and 2-byte start (version 15's; such stores cost version 10's
+// smallest products 0.3 us of 7), else whole 16-byte chunks.
 typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(2)));
-template <typename OutT>
+template <bool kAny, typename OutT>
 __device__ __forceinline__ void store_chunk(OutT* p, const uint4v& v, int left) {
   constexpr int kE = 16 / sizeof(OutT);
-  if (left >= kE) {
+  if constexpr (!kAny) {
+    if (left > 0) *reinterpret_cast<uint4v*>(p) = v;
+  } else if (left >= kE) {
     *reinterpret_cast<uint4u*>(p) = v;
   } else if (left > 0) {
     OutT x[kE];
@@ -650,7 +654,8 @@ struct Epi16<half_t> {
     }
   }
   // The same for a block at (row0, col0) of C that may reach past M rows or
-  // N columns, which are not stored; rows of C start on any 2-byte boundary.
+  // N columns, which are not stored (kAny: see store_chunk).
+  template <bool kAny>
   static __device__ __forceinline__ void flush_edge(uint32_t wbase, half_t* C, int M, int N, int row0, int col0,
                                                     int lane, int half) {
     if (half == 0) return;
@@ -663,7 +668,7 @@ struct Epi16<half_t> {
     for (int q = 0; q < 16; q++) {
       const int row = 8 * q + rsub;
       const uint4v v = epi16_read_pair(wbase, row, ch);
-      if (row0 + row < M) store_chunk(C + (size_t)(row0 + row) * N + col0 + ch * 8, v, left);
+      if (row0 + row < M) store_chunk<kAny>(C + (size_t)(row0 + row) * N + col0 + ch * 8, v, left);
     }
   }
 };
@@ -688,6 +693,7 @@ struct Epi16<float> {
     }
     if (half == 0) wait_lgkmcnt0();  // the region is rewritten by the second half
   }
+  template <bool kAny>
   static __device__ __forceinline__ void flush_edge(uint32_t wbase, float* C, int M, int N, int row0, int col0,
                                                     int lane, int half) {
     const int rsub = lane >> 4, ch = lane & 15;
@@ -697,7 +703,7 @@ struct Epi16<float> {
       const int row = 4 * q + rsub;
       const uint4v v = lds_read16(wbase + row * 256 + 16 * (ch ^ (row & 15)));
       const int r = row0 + half * 64 + row;
-      if (r < M) store_chunk(C + (size_t)r * N + col0 + ch * 4, v, left);
+      if (r < M) store_chunk<kAny>(C + (size_t)r * N + col0 + ch * 4, v, left);
     }
     if (half == 0) wait_lgkmcnt0();
   }
@@ -715,7 +721,7 @@ __device__ __forceinline__ void epilogue16(float4v (&acc)[8][4], uint32_t wbase,
   }
 }
 
-template <typename OutT>
+template <typename OutT, bool kAny>
 __device__ __forceinline__ void epilogue16_edge(float4v (&acc)[8][4], uint32_t wbase, OutT* C, int M, int N,
                                                 int row0, int col0, int lane) {
 #pragma unroll
@@ -724,7 +730,7 @@ __device__ __forceinline__ void epilogue16_edge(float4v (&acc)[8][4], uint32_t w
     for (int i = 4 * half; i < 4 * half + 4; i++)
 #pragma unroll
       for (int j = 0; j < 4; j++) Epi16<OutT>::stage(wbase, lane, i, j, acc[i][j]);
-    Epi16<OutT>::flush_edge(wbase, C, M, N, row0, col0, lane, half);
+    Epi16<OutT>::template flush_edge<kAny>(wbase, C, M, N, row0, col0, lane, half);
   }
 }
 
@@ -1159,7 +1165,7 @@ hipError_t launch_abl(const GemmArgs& a) {
 // the end of a matrix, the A chunks past K are masked, and the C stores skip
 // the chunks outside.  The reference's kernels would launch no blocks for
 // such shapes (matmul_f16_v42_shfl2.cu:124, :520-527).
-template <typename OutT>
+template <typename OutT, bool kAny>
 __global__ __launch_bounds__(kThreads) void f16_pp16_edge_kernel(const half_t* __restrict__ A,
                                                                  const half_t* __restrict__ B,
                                                                  OutT* __restrict__ C, int M, int N, int K, int ldc) {
@@ -1176,25 +1182,32 @@ __global__ __launch_bounds__(kThreads) void f16_pp16_edge_kernel(const half_t* _
 
   float4v acc[8][4];
   pp16_mainloop<true>(A, B, N, K, m0, n0, 0, (K + kBK - 1) / kBK, lds_base, grp, gw, lane, acc, M);
-  epilogue16_edge<OutT>(acc, lds_base + wave * (128 * 64 * 2), C, M, ldc, m0 + grp * 128, n0 + gw * 64,
-                        lane_from_exec());
+  epilogue16_edge<OutT, kAny>(acc, lds_base + wave * (128 * 64 * 2), C, M, kAny ? ldc : N, m0 + grp * 128,
+                              n0 + gw * 64, lane_from_exec());
 }
 
-template <typename OutT>
+// The row pitch of C (other than N, B's, only where B's rows are padded to
+// multiples of 8 and C's are not), and whether its rows start off the 16-byte
+// boundaries.
+int ldc_of(const GemmArgs& a) { return (int)(a.ldc ? a.ldc : a.n); }
+bool any_rows(const GemmArgs& a) { return ldc_of(a) % 8 != 0; }
+
+template <typename OutT, bool kAny>
 hipError_t launch_edge_t(const GemmArgs& a) {
   static std::atomic<uint64_t> attr_done{0};
-  auto kfn = f16_pp16_edge_kernel<OutT>;
+  auto kfn = f16_pp16_edge_kernel<OutT, kAny>;
   hipError_t e = ensure_lds_attr(kfn, kLdsBytes, a.device, attr_done);
   if (e != hipSuccess) return e;
   const int tiles = (int)(((a.m + kBM - 1) / kBM) * ((a.n + kBN - 1) / kBN));
   hipLaunchKernelGGL(kfn, dim3(tiles), dim3(kThreads), kLdsBytes, a.stream,
                      static_cast<const half_t*>(a.A), static_cast<const half_t*>(a.B),
-                     static_cast<OutT*>(a.C), (int)a.m, (int)a.n, (int)a.k, (int)(a.ldc ? a.ldc : a.n));
+                     static_cast<OutT*>(a.C), (int)a.m, (int)a.n, (int)a.k, ldc_of(a));
   return hipGetLastError();
 }
 
+template <bool kAny>
 hipError_t launch_edge(const GemmArgs& a) {
-  return a.out_dtype == VK_DTYPE_F16 ? launch_edge_t<half_t>(a) : launch_edge_t<float>(a);
+  return a.out_dtype == VK_DTYPE_F16 ? launch_edge_t<half_t, kAny>(a) : launch_edge_t<float, kAny>(a);
 }
 
 // Each operand below 2^31 bytes (buffer sizes), and version 7's 32-bit lane
@@ -1259,7 +1272,7 @@ __device__ __forceinline__ bool sk_arrive(float4v (&acc)[8][4], int np, int p, _
 // split tile, the last arrival's sum of all pieces, after which the counter is
 // reset for the next call.  The block starts at row row0, column col0 of C;
 // kEdge: it may reach past M rows or N columns, which are not stored.
-template <typename OutT, bool kEdge, typename PartOff>
+template <typename OutT, bool kEdge, bool kAny, typename PartOff>
 __device__ __forceinline__ void sk_write_c(float4v (&acc)[8][4], int np, int p, __amdgpu_buffer_rsrc_t part,
                                            PartOff part_off, unsigned* cnt, uint32_t wstage, OutT* C, int M,
                                            int N, int row0, int col0) {
@@ -1296,14 +1309,14 @@ __device__ __forceinline__ void sk_write_c(float4v (&acc)[8][4], int np, int p, 
       for (int b = 0; b < 8; b++) Epi16<OutT>::stage(wstage, lane, 2 * bb + (b >> 2), b & 3, t[b]);
     }
     if constexpr (kEdge)
-      Epi16<OutT>::flush_edge(wstage, C, M, N, row0, col0, lane, half);
+      Epi16<OutT>::template flush_edge<kAny>(wstage, C, M, N, row0, col0, lane, half);
     else
       Epi16<OutT>::flush(wstage, C + (size_t)row0 * N + col0, N, lane, half);
   }
   if (np > 1 && lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename OutT, bool kEdge>
+template <typename OutT, bool kEdge, bool kAny>
 __global__ __launch_bounds__(kThreads) void f16_pp16_sk_kernel(const half_t* __restrict__ A,
                                                                const half_t* __restrict__ B,
                                                                OutT* __restrict__ C, int M, int N, int K, int dp,
@@ -1340,8 +1353,8 @@ __global__ __launch_bounds__(kThreads) void f16_pp16_sk_kernel(const half_t* __r
   };
   unsigned* cnt = counters + (size_t)w.tile * kSkWaves + wave;
   if (w.np == 1 || sk_arrive(acc, w.np, w.p, prsrc, part_off, cnt))
-    sk_write_c<OutT, kEdge>(acc, w.np, w.p, prsrc, part_off, cnt, wstage, C, M, kEdge ? ldc : N, m0 + grp * 128,
-                             n0 + gw * 64);
+    sk_write_c<OutT, kEdge, kAny>(acc, w.np, w.p, prsrc, part_off, cnt, wstage, C, M, kAny ? ldc : N,
+                                  m0 + grp * 128, n0 + gw * 64);
 }
 
 // Split-tail plan of a shape: kEdge counts the tiles and k-tiles that reach
@@ -1352,10 +1365,10 @@ SkPlan sk_plan_of(size_t m, size_t n, size_t k, int num_cus) {
   return sk_plan((int64_t)(tm * tn), (int64_t)(kEdge ? (k + kBK - 1) / kBK : k / kBK), num_cus);
 }
 
-template <typename OutT, bool kEdge>
+template <typename OutT, bool kEdge, bool kAny = false>
 hipError_t launch_sk_t(const GemmArgs& a) {
   static std::atomic<uint64_t> attr_done{0};
-  auto kfn = f16_pp16_sk_kernel<OutT, kEdge>;
+  auto kfn = f16_pp16_sk_kernel<OutT, kEdge, kAny>;
   hipError_t e = ensure_lds_attr(kfn, kLdsBytes, a.device, attr_done);
   if (e != hipSuccess) return e;
   const SkPlan p = sk_plan_of<kEdge>(a.m, a.n, a.k, a.num_cus);
@@ -1371,7 +1384,7 @@ hipError_t launch_sk_t(const GemmArgs& a) {
   }
   hipLaunchKernelGGL(kfn, dim3((unsigned)(p.dp + p.units)), dim3(kThreads), kLdsBytes, a.stream,
                      static_cast<const half_t*>(a.A), static_cast<const half_t*>(a.B), static_cast<OutT*>(a.C),
-                     (int)a.m, (int)a.n, (int)a.k, p.dp, p.units, p.pieces, p.chunks, (int)(a.ldc ? a.ldc : a.n), part, counters);
+                     (int)a.m, (int)a.n, (int)a.k, p.dp, p.units, p.pieces, p.chunks, ldc_of(a), part, counters);
   return hipGetLastError();
 }
 
@@ -1382,9 +1395,13 @@ hipError_t launch_sk(const GemmArgs& a) {
 // Version 10: whole tiles with masked edges, or, where the split-tail plan
 // splits (a part-empty last wave, e.g. 1000^3 = 16 tiles), version 9's
 // schedule with the same edges.
+template <bool kAny>
+hipError_t launch_edge_split(const GemmArgs& a) {
+  if (sk_plan_of<true>(a.m, a.n, a.k, a.num_cus).units == 0) return launch_edge<kAny>(a);
+  return a.out_dtype == VK_DTYPE_F16 ? launch_sk_t<half_t, true, kAny>(a) : launch_sk_t<float, true, kAny>(a);
+}
 hipError_t launch_edge_any(const GemmArgs& a) {
-  if (sk_plan_of<true>(a.m, a.n, a.k, a.num_cus).units == 0) return launch_edge(a);
-  return a.out_dtype == VK_DTYPE_F16 ? launch_sk_t<half_t, true>(a) : launch_sk_t<float, true>(a);
+  return any_rows(a) ? launch_edge_split<true>(a) : launch_edge_split<false>(a);
 }
 
 size_t sk_workspace_edge(size_t m, size_t n, size_t k, int num_cus) {
