@@ -32,3 +32,23 @@ def kernel(tmp_path_factory):
 ])
 def test_rows_of_c_in_version_10(kernel, call, name):
     assert name in kernel(*call)
+
+
+# version 11's 64 x 256 tiles (the last template argument) by rounds of the CUs
+@pytest.mark.parametrize("call,wide", [
+    ((F16, 11, 300, 11008, 16384), True),   # 2 -> 1
+    ((F16, 11, 320, 22016, 1024), True),    # 3 -> 2
+    ((F16, 11, 320, 22016, 2048), False),
+    ((F16, 11, 192, 65536, 512), True),     # 4 -> 3
+    ((F16, 11, 192, 65536, 4096), False),
+    ((F16, 11, 320, 65536, 256), True),     # 6 -> 5
+    ((F16, 11, 320, 65536, 2048), False),
+    ((F16, 11, 64, 98304, 4096), True),     # 3 -> 2, half of each square tile empty
+    ((F16, 11, 1024, 4096, 4096), False),   # one round of square tiles
+    ((F16, 11, 256, 16512, 4096), False),   # two rounds either way
+    ((F16, 11, 256, 16512, 64), False),
+    ((F16, 11, 129, 16640, 4096), True),
+])
+def test_wide_tiles_of_version_11(kernel, call, wide):
+    name = kernel(*call)
+    assert ("f16_pp128n_kernel" in name and "ELb0ELb1EE" in name) == wide, name

@@ -561,15 +561,25 @@ hipError_t launch_out(const GemmArgs& a) {
 // A grid of 128 x 128 tiles just past a whole number of rounds of the CUs (258
 // on 256) leaves most of its last round empty; where the 64-row blocks are
 // odd in number, 64 x 256 tiles are fewer.  They take version 13's k-loop over
-// the same sums (bitwise equal).  us per launch, fresh operands, against the
-// square tiles: 300 x 11008 x 4096 (215 for 258) 47.9 / 59.4, 192 x 16640 x 4096
-// (195 for 260) 51.1 / 60.5, 448 x 8712 x 4096 (245 for 276) 55.7 / 68.9.  A
-// 64-deep k-tile takes 0.7 us where a square tile's takes 0.46, so without a
-// round to save the square ones stay (1024 x 4096 x 4096 47.8 / 39.6).
+// the same sums (bitwise equal).  A round of I 64-deep k-tiles takes 2.75 +
+// 0.78 I us with them and 3.4 + 0.44 I with the square ones (fits over 192 to
+// 448 rows, the wide ones' slowest and the square ones' fastest), so a round
+// saved pays from two to one at any depth, from more only while K is small.  us
+// per launch, fresh operands, against the square tiles:
+//   rounds 2 -> 1  300 x 11008 x 4096 46.3 / 57.2, x 16384 176 / 206; 192 x 16640
+//                  x 4096 50.8 / 59.8; 448 x 8712 x 4096 52.0 / 67.2
+//   3 -> 2         320 x 22016 x 1024 30.9 / 31.2, x 2048 54.4 / 51.1
+//   4 -> 3         192 x 65536 x 512 29.6 / 32.8, x 1024 52.5 / 51.9
+//   6 -> 5         320 x 65536 x 256 29.2 / 32.7, x 512 43.7 / 44.2, x 1024 80 / 70
+// Up to 64 rows half of a square tile is empty, and any round saved pays (64 x
+// 98304 x 4096, 3 -> 2, 152 / 158; 64 x 200000 x 2048, 7 -> 4, 167 / 175).
 bool wide_grid(const GemmArgs& a) {
   const size_t c = a.num_cus > 0 ? a.num_cus : 1;
   const size_t square = (a.m + 127) / 128 * ((a.n + 127) / 128), wide = (a.m + 63) / 64 * ((a.n + 255) / 256);
-  return square > c && (wide + c - 1) / c < (square + c - 1) / c;
+  if (square <= c) return false;
+  const size_t rounds_s = (square + c - 1) / c, rounds_w = (wide + c - 1) / c, iters = (a.k + 63) / 64;
+  if (rounds_w >= rounds_s) return false;
+  return a.m <= 64 || rounds_w * (275 + 78 * iters) < rounds_s * (340 + 44 * iters);
 }
 namespace pp128n {
 hipError_t launch_wide(const GemmArgs& a);
