@@ -18,7 +18,10 @@
 //    fragment c holds columns 8(l%16) + c, so a lane's 8 accumulators of a
 //    row are 8 consecutive columns of C and leave as one 16-byte store;
 //  * A comes from the caches into registers as MFMA fragments (16 rows x 64
-//    bytes per load); kD k-steps of both are in flight per wave;
+//    bytes per load); kD k-steps of both are in flight per wave.  Where K is
+//    odd, every other row starts between two dwords, and such loads from 16
+//    rows take half as long again as B's: A is then loaded by whole dwords,
+//    one more per fragment, and shifted;
 //  * the lanes of a last column block that N cuts short take the last 8
 //    columns of the matrix instead (N >= 8): every load stays inside B, and
 //    columns computed twice are the same sum stored twice;
@@ -37,14 +40,13 @@
 // 92.2 / 110 / 191 against 311 / 318 / 316 / 326 (the streaming read alone is
 // 79.4); 16 x 8191 x 8192 29.5 against 127; 128 x 8191 x 8192 55.6 against 131;
 // 16 x 4095 x 4096 13.8 against 59; 64 x 1001 x 1025 15.5 against 33.5; 16 x
-// 301 x 16000 14.5 against 74.
+// 301 x 16000 14.5 against 74.  Odd K, with A shifted in registers and as loaded
+// before: 16 / 64 / 128 x 16391 x 4095 40.5 / 59.7 / 92.6 and 43.2 / 78.0 / 141
+// (copies: 127); 128 x 50256 x 1025 62.9 and 82.3 (65.5).
 #include "vk_device.hpp"
 #include "vk_internal.hpp"
 #include "vk_stream.hpp"
 #include "vk_tile.hpp"
-
-#include <algorithm>
-#include <atomic>
 
 namespace vk {
 namespace {
@@ -58,16 +60,21 @@ constexpr int kMaxRows = 128;
 typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(2)));
 typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// MB 16-row blocks: k-steps in flight per wave, and the workgroups per CU
-// the registers are cut for (256 registers per lane at 2).
-template <int MB>
+// MB 16-row blocks, kOdd: K odd.  k-steps in flight per wave, and the workgroups
+// per CU the registers are cut for (256 registers per lane at 2).
+template <int MB, bool kOdd>
 struct StCfg {
-  static constexpr int kD = MB == 1 ? 3 : MB == 2 ? 2 : 4;
+  static constexpr int kD = MB == 1 ? 3 : MB == 2 ? 2 : MB == 4 && kOdd ? 3 : 4;
   static constexpr int kOcc = MB <= 2 ? 2 : 1;
 };
 
 __device__ __forceinline__ uint4v load16(const char* base, uint32_t off) {
   return *reinterpret_cast<const uint4u*>(base + off);
+}
+
+__device__ __forceinline__ uint4v load16_dwords(const char* base, uint32_t off) {
+  typedef uint32_t uint4d __attribute__((ext_vector_type(4), aligned(4)));
+  return *reinterpret_cast<const uint4d*>(base + off);
 }
 
 // The low (kHi = false) or high halves of two dwords: {lo, hi} of the result.
@@ -87,11 +94,11 @@ __device__ __forceinline__ void store_row8(float* p, const float4v (&x)[2]) {
   *reinterpret_cast<float4u*>(p + 4) = x[1];
 }
 
-template <int MB, typename OutT>
-__global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
+template <int MB, typename OutT, bool kOdd>
+__global__ __launch_bounds__(kThreads, (StCfg<MB, kOdd>::kOcc)) void f16_stream_kernel(
     const half_t* __restrict__ A, const half_t* __restrict__ B, OutT* __restrict__ C, int M, int N, int K, int ks,
     int halves, float* __restrict__ part, unsigned* __restrict__ counters) {
-  constexpr int D = StCfg<MB>::kD;
+  constexpr int D = StCfg<MB, kOdd>::kD;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, i16 = lane & 15;
@@ -130,6 +137,7 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
 
   struct Step {
     uint4v b[8], a[MB];
+    uint32_t next[kOdd ? MB : 1];  // kOdd: the dword that an odd row's fragment ends in
   };
   Step buf[D];
   auto load = [&](Step& s, int j) {
@@ -138,7 +146,27 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
 #pragma unroll
     for (int i = 0; i < 8; i++) s.b[i] = load16(pb, offB[i]);
 #pragma unroll
-    for (int r = 0; r < MB; r++) s.a[r] = load16(pa, offA[r]);
+    for (int r = 0; r < MB; r++) {
+      if constexpr (kOdd) {
+        // the last dword once more for an even row, whose fragment may be the
+        // end of A
+        s.a[r] = load16_dwords(pa, offA[r] & ~3u);
+        s.next[r] = *reinterpret_cast<const uint32_t*>(pa + ((offA[r] + 14) & ~3u));
+      } else {
+        s.a[r] = load16(pa, offA[r]);
+      }
+    }
+  };
+  // The fragments of A in a loaded step.
+  auto shift_a = [&](Step& s) {
+    if constexpr (kOdd)
+#pragma unroll
+      for (int r = 0; r < MB; r++) {
+        const uint32_t sh = (offA[r] & 2u) * 8u;
+#pragma unroll
+        for (int d = 0; d < 4; d++)
+          s.a[r][d] = __builtin_amdgcn_alignbit(d < 3 ? s.a[r][d + 1] : s.next[r], s.a[r][d], sh);
+      }
   };
   auto multiply = [&](const Step& s) {
 #pragma unroll
@@ -166,6 +194,7 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
 #pragma unroll
     for (int u = 0; u < D; u++) {
       __builtin_amdgcn_sched_barrier(0);
+      shift_a(buf[u]);
       multiply(buf[u]);
       __builtin_amdgcn_sched_barrier(0);
       load(buf[u], s0 + u + D);
@@ -174,12 +203,18 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
   // fewer than 2 D steps left (the loop above asks no step whether it exists)
 #pragma unroll
   for (int u = 0; u < D; u++) {
-    if (s0 + u < ns) multiply(buf[u]);
+    if (s0 + u < ns) {
+      shift_a(buf[u]);
+      multiply(buf[u]);
+    }
     if (s0 + u + D < ns) load(buf[u], s0 + u + D);
   }
 #pragma unroll
   for (int u = 0; u < D; u++)
-    if (s0 + u + D < ns) multiply(buf[u]);
+    if (s0 + u + D < ns) {
+      shift_a(buf[u]);
+      multiply(buf[u]);
+    }
   if (p == parts - 1 && tsteps * kKStep < K) {
     const int kt = tsteps * kKStep + 8 * g;
     const int past = max(kt + 8 - K, 0);  // of the lane's 8 k, how many lie past K
@@ -216,7 +251,7 @@ __global__ __launch_bounds__(kThreads, StCfg<MB>::kOcc) void f16_stream_kernel(
 int halves_of(size_t m) { return m > 64 ? 2 : 1; }
 int blocks_of(size_t m) { return (int)(((m + 15) / 16 + halves_of(m) - 1) / halves_of(m)); }
 
-template <int MB, typename OutT>
+template <int MB, typename OutT, bool kOdd>
 hipError_t launch_t(const GemmArgs& a, size_t ws_limit) {
   const int halves = halves_of(a.m);
   const int ks = f16_stream_pieces(a.m, a.n, a.k, ws_limit, a.num_cus);
@@ -225,15 +260,19 @@ hipError_t launch_t(const GemmArgs& a, size_t ws_limit) {
   const hipError_t e = stream_buffers(a, ks, counters, part);
   if (e != hipSuccess) return e;
   const unsigned grid = (unsigned)((a.n + kNC - 1) / kNC * ks * halves);
-  hipLaunchKernelGGL((f16_stream_kernel<MB, OutT>), dim3(grid), dim3(kThreads), 0, a.stream,
+  hipLaunchKernelGGL((f16_stream_kernel<MB, OutT, kOdd>), dim3(grid), dim3(kThreads), 0, a.stream,
                      static_cast<const half_t*>(a.A), static_cast<const half_t*>(a.B), static_cast<OutT*>(a.C),
                      (int)a.m, (int)a.n, (int)a.k, ks, halves, part, counters);
   return hipGetLastError();
 }
 
+template <int MB, bool kOdd>
+hipError_t launch_out(const GemmArgs& a, size_t ws_limit) {
+  return a.out_dtype == VK_DTYPE_F16 ? launch_t<MB, half_t, kOdd>(a, ws_limit) : launch_t<MB, float, kOdd>(a, ws_limit);
+}
 template <int MB>
 hipError_t launch_mb(const GemmArgs& a, size_t ws_limit) {
-  return a.out_dtype == VK_DTYPE_F16 ? launch_t<MB, half_t>(a, ws_limit) : launch_t<MB, float>(a, ws_limit);
+  return a.k % 2 && a.m > 1 ? launch_out<MB, true>(a, ws_limit) : launch_out<MB, false>(a, ws_limit);
 }
 
 }  // namespace
