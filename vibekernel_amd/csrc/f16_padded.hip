@@ -137,7 +137,9 @@ hipError_t launch_padded(const GemmArgs& a) {
   }
   if (L.pad_b) {
     b.B = ws + L.b_off;
-    e = repitch(a.B, ws + L.b_off, a.k, a.n, L.k8, L.n8, a.stream);
+    // rows that only follow each other (N a multiple of 8) are one long row
+    e = L.n8 == a.n ? repitch(a.B, ws + L.b_off, 1, a.k * a.n, 1, L.k8 * L.n8, a.stream)
+                    : repitch(a.B, ws + L.b_off, a.k, a.n, L.k8, L.n8, a.stream);
     if (e != hipSuccess) return e;
   }
   b.workspace = L.inner ? ws : nullptr;
