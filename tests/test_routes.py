@@ -61,3 +61,26 @@ def test_wide_tiles_of_version_11(kernel, call, wide):
                                        ((F16, 15, 128, 4096, 4095), "f16_stream_kernelILi4EDF16_Lb1EE")])
 def test_odd_k_of_few_rows(kernel, call, name):
     assert name in kernel(*call)
+
+
+# version 15 through registers or through copies and version 10
+@pytest.mark.parametrize("call,name", [
+    ((F16, 15, 1000, 1001, 999), "f16_any"),
+    ((F16, 15, 700, 700, 10239), "f16_any"),       # few tiles: K up to 10240
+    ((F16, 15, 700, 700, 10241), "f16_pp16"),
+    ((F16, 15, 300, 200, 1023), "f16_any"),        # fewer still: K up to 1024
+    ((F16, 15, 300, 200, 4095), "f16_pp16"),
+    ((F16, 15, 128, 50001, 1023), "f16_any"),      # half-empty 256 x 256 tiles
+    ((F16, 15, 100000, 65, 513), "f16_any"),
+    ((F16, 15, 1000, 8001, 1023), "f16_any"),      # two 128 x 128 tiles per CU
+    ((F16, 15, 1500, 3001, 1801), "f16_pp16"),
+    ((F16, 15, 50000, 304, 191), "f16_any"),       # few columns
+    ((F16, 15, 50000, 304, 257), "f16_pp16"),
+    ((F16, 15, 50000, 400, 65), "f16_pp16"),
+    ((F16, 15, 300, 50000, 129), "f16_any"),       # few rows, aligned columns
+    ((F16, 15, 300, 50001, 129), "f16_pp16"),
+    ((F16, 15, 4096, 8192, 255), "f16_pp16"),
+    ((F16, 15, 2049, 2051, 2052), "f16_pp16"),     # past 2^33
+])
+def test_copies_of_version_15(kernel, call, name):
+    assert name in kernel(*call)

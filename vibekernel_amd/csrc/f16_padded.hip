@@ -5,9 +5,9 @@
 // every row must start on a 16-byte boundary: N and K multiples of 8.  Other
 // shapes (a vocabulary of 50,257 columns, K = 4095) take one of three ways:
 //  * up to 128 rows with K >= 1024: f16_stream.hip reads B once;
-//  * up to 2^33 multiply-adds: f16_any.hip loads any alignment through
-//    registers (no_copies below);
-//  * larger ones run version 10 (any M; N and K multiples of 8) on row-padded
+//  * products that cannot earn copies back: f16_any.hip loads any alignment
+//    through registers (no_copies below);
+//  * the others run version 10 (any M; N and K multiples of 8) on row-padded
 //    copies in the workspace: A (M x K) with row pitch K8 = K rounded up to 8
 //    when K % 8 != 0, B (K x N) with pitch N8 and K8 rows when N % 8 or K % 8
 //    != 0, the pads zero (A's pad columns meet B's pad rows: zero times zero).
@@ -64,16 +64,18 @@ PadLayout layout_of(size_t m, size_t n, size_t k, int num_cus) {
 // dst (drows rows of dpitch elements, a multiple of 8) <- src (rows rows of
 // width elements), the elements past width or rows zero.  Each thread copies
 // one 16-byte chunk of kRows consecutive destination rows, its loads out
-// together; adjacent threads take adjacent chunks.  A chunk inside its source
-// row is one 16-byte load at any 2-byte address, one at the row's end single
-// elements.
-constexpr int kRows = 4;
+// together; adjacent threads take adjacent chunks, and a workgroup as many
+// threads per row as the row has chunks to give them (a power of two).  A chunk
+// inside its source row is one 16-byte load at any 2-byte address, one at the
+// row's end single elements.
 typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(2)));
+template <int kRows>
 __global__ __launch_bounds__(256) void repitch_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
                                                       int rows, int width, int drows, int dpitch) {
-  const int col = 8 * (int)(blockIdx.x * 256 + threadIdx.x);
+  const int col = 8 * (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (col >= dpitch) return;
-  for (int r0 = (int)blockIdx.y * kRows; r0 < drows; r0 += (int)gridDim.y * kRows) {
+  for (int r0 = (int)(blockIdx.y * blockDim.y + threadIdx.y) * kRows; r0 < drows;
+       r0 += (int)(gridDim.y * blockDim.y) * kRows) {
     uint4v v[kRows];
 #pragma unroll
     for (int i = 0; i < kRows; i++) {
@@ -95,27 +97,62 @@ __global__ __launch_bounds__(256) void repitch_kernel(const uint16_t* __restrict
   }
 }
 
-hipError_t repitch(const void* src, void* dst, size_t rows, size_t width, size_t drows, size_t dpitch,
-                   hipStream_t s) {
-  const unsigned gx = (unsigned)((dpitch / 8 + 255) / 256);
-  const unsigned gy = (unsigned)std::min<size_t>((drows + kRows - 1) / kRows, 65535);
-  hipLaunchKernelGGL(repitch_kernel, dim3(gx, gy), dim3(256), 0, s, static_cast<const uint16_t*>(src),
+template <int kRows>
+hipError_t repitch_rows(const void* src, void* dst, size_t rows, size_t width, size_t drows, size_t dpitch,
+                        hipStream_t s) {
+  unsigned tx = 256;  // threads per row
+  while (tx > 1 && tx / 2 >= dpitch / 8) tx /= 2;
+  const unsigned ty = 256 / tx;
+  const unsigned gx = (unsigned)((dpitch / 8 + tx - 1) / tx);
+  const unsigned gy = (unsigned)std::min<size_t>((drows + kRows * ty - 1) / (kRows * ty), 65535);
+  hipLaunchKernelGGL(repitch_kernel<kRows>, dim3(gx, gy), dim3(tx, ty), 0, s, static_cast<const uint16_t*>(src),
                      static_cast<uint16_t*>(dst), (int)rows, (int)width, (int)drows, (int)dpitch);
   return hipGetLastError();
+}
+// 4 rows per thread where that leaves 4 workgroups per CU or more (a 4000 x 33 A:
+// 3.2 us with 4, 2.0 with 1).
+hipError_t repitch(const void* src, void* dst, size_t rows, size_t width, size_t drows, size_t dpitch,
+                   hipStream_t s) {
+  const bool many = drows >= 4 && drows * (dpitch / 8) >= ((size_t)1 << 20);
+  return many ? repitch_rows<4>(src, dst, rows, width, drows, dpitch, s)
+              : repitch_rows<1>(src, dst, rows, width, drows, dpitch, s);
 }
 
 // Few rows need no copies: f16_stream.hip reads B once at any row alignment.
 bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_stream_takes(m, n, k); }
 
-// Neither do products too small to earn the copies back (f16_any.hip).  us per
-// launch against the copies and version 10: 1000 x 1001 x 999 13.5 / 33, 300 x
-// 4095 x 4096 44 / 58, 2000 x 2001 x 2002 (2^33) 51 / 56, but 700 x 8191 x 2048
-// 64 / 61, 300 x 11007 x 4096 92 / 98 and 4096 x 4095 x 4096 260 / 124.  A few
-// tiles of a deep K keep version 10's split sum (300 x 200 x 4095: 28.7 / 49).
+// Neither do products that cannot earn the copies back (f16_any.hip), up to 2^33
+// multiply-adds.  us per launch, f16_any.hip / copies and version 10:
+//  * while 64 x 64 tiles are at most 4 per CU (f16_any_launch's rule for them): 1000
+//    x 1001 x 1023 13.0 / 34.3, 2000 x 2001 x 2001 48 / 55; but a workgroup's
+//    k-loop is one chain, which the copies' split sum cuts in 8: 700 x 700 x 8191
+//    49.6 / 61, x 12287 77 / 79, x 16383 105 / 90 (200 x 500 x 32767 215 against
+//    129), and a few tiles of K > 1024 are slower from the start (300 x 200 x
+//    4095 28.7 / 49 with 20 tiles of 4095, 160 CUs idle);
+//  * where half of each 256 x 256 tile is empty: 128 x 50001 x 1023 53 / 67, 100000
+//    x 65 x 513 63 / 79;
+//  * while 128 x 128 tiles are at most 2 per CU, up to K = 1024: 1000 x 8001 x 129
+//    18.4 / 20.4, 3000 x 1500 x 1023 35 / 40, 1500 x 3001 x 1801 63 / 52;
+//  * past that few columns up to K = 256, whose copy of A is most of the work:
+//    50000 x 304 x 193 32 / 36, x 257 47 / 43, 50000 x 200 x 193 24 / 29, x 385 45 /
+//    39, 30000 x 600 x 129 28.0 / 29.6; 50000 x 400 x 65 28.7 / 26.3; and few rows of whole 8-column chunks: 300 x
+//    50000 x 193 32 / 35, x 257 47 / 40; 300 x 50001 x 65 30.3 / 29.5, 400 x 50000 x
+//    65 31.5 / 26.3, 129 x 100000 x 129 38.7 / 34.0;
+//  * the rest take the copies: 4000 x 4000 x 33 18.6 / 15.3, 4096 x 8192 x 255 55 /
+//    40, 8192 x 8193 x 65 111 / 59.
 bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
-  const size_t tiles = (m + 63) / 64 * ((n + 63) / 64);
-  if ((m + 127) / 128 > 65535) return false;  // rows of its tiles are grid.y
-  return (n % 8 || k % 8) && m * n * k <= ((size_t)1 << 33) && (8 * tiles >= (size_t)num_cus || k <= 1024);
+  if (n % 8 == 0 && k % 8 == 0) return false;           // no copies to make
+  if ((m + 127) / 128 > 65535) return false;            // rows of its tiles are grid.y
+  if (m * n * k > (size_t)1 << 33) return false;
+  const size_t c = num_cus;
+  auto tiles = [&](size_t t) { return (m + t - 1) / t * ((n + t - 1) / t); };
+  if (tiles(64) <= 4 * c) return k <= 1024 || (8 * tiles(64) >= c && k <= 10240);
+  if (m <= 128 || n <= 128) return true;
+  if (tiles(128) <= 2 * c) return k <= 1024;
+  const size_t filled = 100 * m * n / (tiles(256) * 65536);  // per cent of the 256 x 256 tiles
+  const bool few = tiles(128) <= 5 * c;
+  if (k > 256) return false;
+  return m > n ? n <= 256 || filled <= (few ? 80 : 60) : n % 8 == 0 && k > 64 && filled <= 60 && few;
 }
 
 hipError_t launch_padded(const GemmArgs& a) {
