@@ -38,7 +38,23 @@ def test_bits_equal_to_the_oracle(gpu, oracle, shape, shift):
     assert np.array_equal(C.cpu().numpy(), oracle.sgemm(A, B))
 
 
-@pytest.mark.parametrize("shape", [(3, 5, 35), (70, 67, 130)])
+# K within one k-tile of 32 or 64, two of 64, and any K with N below 4: at the
+# 16-deep groups and the 16-row blocks that are left out when they hold nothing
+@pytest.mark.parametrize("mn", [(1, 5), (16, 3), (17, 16), (33, 67), (48, 17), (70, 130)], ids=lambda mn: "%dx%d" % mn)
+@pytest.mark.parametrize("shift", [0, 1])
+def test_small_k(gpu, oracle, mn, shift):
+    m, n = mn
+    for k in (1, 2, 3, 4, 5, 15, 16, 17, 31, 32, 33, 48, 50, 63, 64, 65, 80, 83, 112, 127, 128):
+        test_bits_equal_to_the_oracle(gpu, oracle, (m, n, k), shift)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 129), (64, 3, 192), (65, 2, 200), (47, 3, 257), (130, 1, 1023)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_few_columns(gpu, oracle, shape, shift):
+    test_bits_equal_to_the_oracle(gpu, oracle, shape, shift)
+
+
+@pytest.mark.parametrize("shape", [(3, 5, 35), (70, 67, 130), (70, 67, 30), (18, 40, 61), (34, 65, 100), (33, 2, 200)])
 def test_values_past_the_edges_never_reach_c(gpu, shape):
     """A[1][0] is what row 0 reads past K, B[k-1][0] what row k-2 reads past
     N: infinite, they may only reach row 1 and column 0."""

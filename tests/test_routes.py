@@ -84,3 +84,19 @@ def test_odd_k_of_few_rows(kernel, call, name):
 ])
 def test_copies_of_version_15(kernel, call, name):
     assert name in kernel(*call)
+
+
+# fp32 version 1 off its asm kernel: tile rows / 64, k-tile depth, k-tiles (0: any number, 3: any, N below 4)
+@pytest.mark.parametrize("call,name", [
+    ((F32, 1, 1000, 1001, 32), "f32_any_kernelILi1ELi32ELi1EE"),
+    ((F32, 1, 1000, 1001, 33), "f32_any_kernelILi1ELi64ELi1EE"),
+    ((F32, 1, 1000, 1001, 64), "f32_any_kernelILi1ELi64ELi1EE"),
+    ((F32, 1, 1000, 1001, 65), "f32_any_kernelILi1ELi64ELi2EE"),
+    ((F32, 1, 1000, 1001, 128), "f32_any_kernelILi1ELi64ELi2EE"),
+    ((F32, 1, 1000, 1001, 129), "f32_any_kernelILi1ELi64ELi0EE"),
+    ((F32, 1, 1000, 3, 129), "f32_any_kernelILi1ELi64ELi3EE"),
+    ((F32, 1, 1000, 3, 128), "f32_any_kernelILi1ELi64ELi2EE"),
+    ((F32, 1, 1990, 2047, 33), "f32_any_kernelILi2ELi32ELi0EE"),
+])
+def test_small_k_of_fp32_version_1(kernel, call, name):
+    assert name in kernel(*call)
