@@ -177,8 +177,16 @@ hipError_t launch_mb(const GemmArgs& a, size_t ws_limit) {
 // 4096 x 4096 / 8192 x 8192 13.4 / 21.1 / 28.5 / 79 against 10.8 / 17.6 / 31.7 /
 // 98.8.  What bounds the large ones is the read of B (16 x 8192 x 8192: 5.0
 // TB/s), the small ones the launch and the pieces' hand-off.
+// Where K is one to three of the tiles' whole 32-deep k-tiles, the waves have a
+// step or two each and their sum is most of the time, so the tiles keep a grid of
+// up to one column block per CU (two from 17 rows) and, for 64 rows, the largest
+// ones: 32 x 16384 x 64 / 96 4.8 / 5.5 us against 4.4 / 4.9, 32 x 20000 x 64 6.8 /
+// 5.5, 64 x 262144 x 64 56.3 / 51.6; but 16 x 20000 x 96 6.2 / 6.4, 32 x 32768 x 64
+// 7.3 / 9.0, 64 x 262144 x 128 72 / 79.
 bool f32_stream_takes(size_t m, size_t n, size_t k) {
   if (m > 32 && n * k < ((size_t)1 << 23)) return false;
+  if (k % 32 == 0 && m <= 32 && k <= 96 && n <= (m <= 16 ? 16384 : 32767)) return false;
+  if (k % 32 == 0 && m > 56 && k <= 64) return false;
   return m >= 1 && m <= kMaxRows && n >= 4 && n % 4 == 0 && n < (1u << 25) && k >= 4 && k % 4 == 0 && k < (1u << 23);
 }
 
