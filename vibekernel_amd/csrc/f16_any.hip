@@ -91,7 +91,7 @@ __global__ __launch_bounds__(kThreads, 2) void f16_any_kernel(const half_t* __re
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int tm, tn;
-  tile_of((int)(blockIdx.y * gridDim.x + blockIdx.x), tiles_m, tiles_n, tm, tn);
+  tile_of((int)(blockIdx.y * (unsigned)tiles_n + blockIdx.x), tiles_m, tiles_n, tm, tn);
   const int64_t m0 = (int64_t)tm * T, n0 = (int64_t)tn * T;
   const uint32_t lbase = lds_addr32(lds);  // A of buffers 0, 1, then B of buffers 0, 1
 

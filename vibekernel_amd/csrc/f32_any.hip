@@ -101,7 +101,7 @@ __device__ __forceinline__ float4v cut_fix(const float4v& v, int64_t valid) {
 template <int NB, int kDeep, int kTiles>
 __global__ __launch_bounds__(kThreads, NB == 1 ? 4 : 2) void f32_any_kernel(const float* __restrict__ A, const float* __restrict__ B,
                                                               float* __restrict__ C, int64_t M, int64_t N, int64_t K,
-                                                              int tiles_m, int tiles_n) {
+                                                              int tiles_m, int tiles_n, int grid_x) {
   using G = AnyCfg<NB, kDeep, kTiles>;
   constexpr int T = G::kT, BK = G::kBK, P = G::kPitchA, L = G::kLd, RB = G::kRB, CB = G::kCB;
   __shared__ __attribute__((aligned(16))) float As[G::kBufs][4 * G::kQuarterA];
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kThreads, NB == 1 ? 4 : 2) void f32_any_kernel(cons
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, l16 = lane & 15;
-  const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+  const int id = (int)(blockIdx.y * (unsigned)grid_x + blockIdx.x);
   if (id >= tiles_m * tiles_n) return;  // the last row of a folded grid
   int tm, tn;
   tile_of(id, tiles_m, tiles_n, tm, tn);
@@ -340,7 +340,7 @@ hipError_t launch_any(const GemmArgs& a) {
   const size_t gx = std::min(tn, (((size_t)1 << 32) - 1) / kThreads), gy = gx == tn ? tm : (tm * tn + gx - 1) / gx;
   hipLaunchKernelGGL((f32_any_kernel<NB, kDeep, kTiles>), dim3((unsigned)gx, (unsigned)gy), dim3(kThreads), 0, a.stream,
                      static_cast<const float*>(a.A), static_cast<const float*>(a.B), static_cast<float*>(a.C),
-                     (int64_t)a.m, (int64_t)a.n, (int64_t)a.k, (int)tm, (int)tn);
+                     (int64_t)a.m, (int64_t)a.n, (int64_t)a.k, (int)tm, (int)tn, (int)gx);
   return hipGetLastError();
 }
 
