@@ -51,6 +51,16 @@ def test_random_and_integer(gpu, oracle, shape, out, shift):
         assert np.array_equal(_run(A, B, out, shift).astype(np.float64), A.astype(np.float64) @ B.astype(np.float64))
 
 
+# C in whole rows through LDS or not, at both sides of half a tile; 128 x 128 tiles from (63, 65603, 9) on
+@pytest.mark.parametrize("shape", [(31, 33, 40), (32, 31, 40), (32, 33, 40), (33, 39, 7), (95, 41, 70), (63, 65603, 9),
+                                   (64, 65603, 9), (70001, 63, 9), (70001, 65, 9), (65, 65543, 5)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_rows_of_c(gpu, oracle, shape, shift):
+    m, n, k = shape
+    A, B = make_inputs(m, n, k, "int", seed=m + n + k)  # sums of at most 4 k: exact in fp16
+    assert np.array_equal(_run(A, B, "f16", shift).astype(np.float32), A.astype(np.float32) @ B.astype(np.float32))
+
+
 @pytest.mark.parametrize("shape", [(3, 5, 35), (70, 67, 130), (1700, 1603, 260)])
 def test_values_past_the_edges_never_reach_c(gpu, shape):
     """A[1][0] is what row 0 reads past K, B[k-1][0] what row k-2 reads past

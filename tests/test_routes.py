@@ -112,3 +112,20 @@ def test_small_k_of_fp32_version_1(kernel, call, name):
 ])
 def test_few_rows_of_fp32_version_3(kernel, call, name):
     assert name in kernel(*call)
+
+
+# fp16 version 1: tile rows / 64, N or K below 8, C in whole rows
+@pytest.mark.parametrize("call,name", [
+    ((F16, 1, 32, 33, 40), "f16_any_kernelILi1EDF16_Lb0ELb1EE"),
+    ((F16, 1, 31, 33, 40), "f16_any_kernelILi1EDF16_Lb0ELb0EE"),
+    ((F16, 1, 32, 31, 40), "f16_any_kernelILi1EDF16_Lb0ELb0EE"),
+    ((F16, 1, 33, 39, 7), "f16_any_kernelILi1EDF16_Lb1ELb1EE"),
+    ((F16, 1, 64, 65603, 9), "f16_any_kernelILi2EDF16_Lb0ELb1EE"),
+    ((F16, 1, 63, 65603, 9), "f16_any_kernelILi2EDF16_Lb0ELb0EE"),
+    ((F16, 1, 70001, 65, 9), "f16_any_kernelILi2EDF16_Lb0ELb1EE"),
+    ((F16, 1, 70001, 63, 9), "f16_any_kernelILi2EDF16_Lb0ELb0EE"),
+    ((F16, 1, 4000, 4002, 9), "f16_any_kernelILi2EDF16_Lb0ELb0EE"),
+    ((F16, 1, 4000, 4001, 9), "f16_any_kernelILi2EDF16_Lb0ELb1EE"),
+])
+def test_rows_of_c_in_fp16_version_1(kernel, call, name):
+    assert name in kernel(*call)

@@ -57,7 +57,17 @@ typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t uint2u __attribute__((ext_vector_type(2), aligned(2)));
 typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// 4 consecutive columns of C, `valid` of them inside the matrix.
+// 8 or 4 consecutive columns of C, `valid` of them inside the matrix.
+__device__ __forceinline__ void store8(half_t* p, const uint4v& v, int64_t valid) {
+  if (valid >= 8) {
+    *reinterpret_cast<uint4u*>(p) = v;
+  } else {
+    const half8 h = __builtin_bit_cast(half8, v);
+#pragma unroll
+    for (int c = 0; c < 7; c++)
+      if (c < valid) p[c] = h[c];
+  }
+}
 __device__ __forceinline__ void store4(half_t* p, const float4v& v, int64_t valid) {
   const half4 h = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
   if (valid >= 4) {
@@ -79,8 +89,8 @@ __device__ __forceinline__ void store4(float* p, const float4v& v, int64_t valid
   }
 }
 
-// kNarrow: N or K below 8.
-template <int NB, typename OutT, bool kNarrow>
+// kNarrow: N or K below 8.  kRows: C in whole rows of the wave's block (fp16).
+template <int NB, typename OutT, bool kNarrow, bool kRows>
 __global__ __launch_bounds__(kThreads, 2) void f16_any_kernel(const half_t* __restrict__ A,
                                                               const half_t* __restrict__ B, OutT* __restrict__ C,
                                                               int64_t M, int64_t N, int64_t K, int tiles_m,
@@ -268,30 +278,63 @@ __global__ __launch_bounds__(kThreads, 2) void f16_any_kernel(const half_t* __re
   }
 
   // Block (i, j), register r, lane l: row 16 i + l % 16, column 16 j + 4 (l / 16) + r.
+  if constexpr (kRows) {
+    // Through LDS, in units of 4 columns, unit ^ row.
+    constexpr int kUnits = 8 * NB, kRow = 8 * kUnits;  // units and bytes per row of the block
+    __syncthreads();  // every wave is done with the k-tiles
+    const uint32_t base = lbase + wave * (32 * NB * kRow);
 #pragma unroll
-  for (int i = 0; i < NBk; i++) {
-    const int64_t row = m0 + wr + 16 * i + l16;
+    for (int i = 0; i < NBk; i++)
 #pragma unroll
-    for (int j = 0; j < NBk; j++) {
-      const int64_t col = n0 + wc + 16 * j + 4 * g;
-      if (row < M && col < N) store4(C + row * N + col, acc[i][j], N - col);
+      for (int j = 0; j < NBk; j++) {
+        const int row = 16 * i + l16;
+        const half4 h = {(half_t)acc[i][j][0], (half_t)acc[i][j][1], (half_t)acc[i][j][2], (half_t)acc[i][j][3]};
+        lds_write8(base + row * kRow + 8 * ((4 * j + g) ^ (row & (kUnits - 1))), h);
+      }
+    constexpr int kLanes = kUnits / 2;  // per row, 8 columns each
+#pragma unroll
+    for (int q = 0; q < 32 * NB * kLanes / 64; q++) {
+      const int row = q * (64 / kLanes) + lane / kLanes, c = lane % kLanes;
+      const uint4v x = lds_read16(base + row * kRow + 16 * (c ^ ((row & (kUnits - 1)) >> 1)));
+      const uint4v v = row & 1 ? uint4v{x[2], x[3], x[0], x[1]} : x;
+      const int64_t r = m0 + wr + row, col = n0 + wc + 8 * c;
+      if (r < M) store8(reinterpret_cast<half_t*>(C) + r * N + col, v, N - col);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NBk; i++) {
+      const int64_t row = m0 + wr + 16 * i + l16;
+#pragma unroll
+      for (int j = 0; j < NBk; j++) {
+        const int64_t col = n0 + wc + 16 * j + 4 * g;
+        if (row < M && col < N) store4(C + row * N + col, acc[i][j], N - col);
+      }
     }
   }
 }
 
-template <int NB, typename OutT>
+template <int NB, typename OutT, bool kRows>
 hipError_t launch_t(const GemmArgs& a) {
   const size_t tm = (a.m + AnyCfg<NB>::kT - 1) / AnyCfg<NB>::kT, tn = (a.n + AnyCfg<NB>::kT - 1) / AnyCfg<NB>::kT;
-  auto kfn = a.n < 8 || a.k < 8 ? f16_any_kernel<NB, OutT, true> : f16_any_kernel<NB, OutT, false>;
+  auto kfn = a.n < 8 || a.k < 8 ? f16_any_kernel<NB, OutT, true, kRows> : f16_any_kernel<NB, OutT, false, kRows>;
   hipLaunchKernelGGL(kfn, dim3((unsigned)tn, (unsigned)tm), dim3(kThreads), 0, a.stream,
                      static_cast<const half_t*>(a.A), static_cast<const half_t*>(a.B), static_cast<OutT*>(a.C),
                      (int64_t)a.m, (int64_t)a.n, (int64_t)a.k, (int)tm, (int)tn);
   return hipGetLastError();
 }
 
+// An fp16 C with an odd number of columns leaves in whole rows of a wave's block
+// where at least half of a tile's rows and more than half of its
+// columns are there; straight from the registers a row gets 32 bytes at a time.  us
+// per launch, rows / straight: 8192 x 8191 x 16 53.7 / 91.7, 4000 x 4001 x 1 15.2 /
+// 21.2, 128 x 50001 x 65 11.6 / 14.0; 1 x 1048577 x 65 129.7 / 121.6; an even
+// number 8192 x 8190 x 1 46 / 53, 50000 x 130 x 65 18.3 / 17.2, 3000 x 1500 x 193 14.3 /
+// 13.5.  (Both in one kernel spill more: 1 x 1048577 x 65 131.3.)
 template <int NB>
 hipError_t launch_nb(const GemmArgs& a) {
-  return a.out_dtype == VK_DTYPE_F16 ? launch_t<NB, half_t>(a) : launch_t<NB, float>(a);
+  if (a.out_dtype != VK_DTYPE_F16) return launch_t<NB, float, false>(a);
+  const bool rows = a.n % 2 != 0 && 2 * a.m >= (size_t)AnyCfg<NB>::kT && 2 * a.n > (size_t)AnyCfg<NB>::kT;
+  return rows ? launch_t<NB, half_t, true>(a) : launch_t<NB, half_t, false>(a);
 }
 
 // grid.y, rows of 128-row tiles at least, holds up to 65535.
