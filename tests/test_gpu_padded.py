@@ -1,8 +1,9 @@
-"""GPU parity of version 15 -- any fp16 shape through row-padded copies of
-A, B and C around version 10 -- through the C ABI.
+"""GPU parity of version 15 -- any fp16 shape, through row-padded copies of A
+and B around version 10 or without them -- through the C ABI.
 
 * Its results are version 10's on explicitly zero-padded operands (N and K
-  rounded up to 8), bit for bit: the pad only adds exact zeros.
+  rounded up to 8), bit for bit: the pad only adds exact zeros.  (Few rows have
+  a sum order of their own: tests/test_gpu_stream.py.)
 * Random inputs: within the fp32 accumulation bound of the exact (fp64)
   product (plus fp16 rounding for fp16 output); integer inputs exact.
 * Nothing outside C is written (NaN guards before and after it).
@@ -18,6 +19,10 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(1000, 1001, 1000), (999, 1000, 1001), (17, 33, 65), (1, 1, 1), (257, 4095, 136), (64, 50257, 512),
           (300, 200, 4095), (1024, 1024, 1023)]
+# through the copies, N off the multiples of 8 (C rows at any alignment): split
+# sums, whole tiles, K a multiple of 8 or not, fewer than 16 columns
+COPIES = [(300, 201, 4095), (129, 9, 4097), (700, 700, 10249), (2049, 2051, 2052), (4096, 4095, 1032), (4000, 4001, 33),
+          (4000, 4003, 40)]
 
 
 def _padded(A, B):
@@ -31,7 +36,7 @@ def _padded(A, B):
     return Ap, Bp
 
 
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape", SHAPES + COPIES)
 @pytest.mark.parametrize("out", ["f16", "f32"])
 def test_random_vs_exact_and_v10_padded(gpu, oracle, shape, out):
     m, n, k = shape
@@ -45,7 +50,8 @@ def test_random_vs_exact_and_v10_padded(gpu, oracle, shape, out):
     assert np.array_equal(np.ascontiguousarray(C).view(u), np.ascontiguousarray(C10).view(u))
 
 
-@pytest.mark.parametrize("shape", [(300, 261, 77), (1, 9, 7), (130, 1001, 1030)])
+@pytest.mark.parametrize("shape", [(300, 261, 77), (1, 9, 7), (130, 1001, 1030), (129, 9, 4097), (300, 201, 4095),
+                                   (4000, 4001, 33), (4000, 4003, 40)])
 @pytest.mark.parametrize("out", ["f16", "f32"])
 def test_integer_exact_and_writes_only_c(gpu, shape, out):
     import torch
@@ -69,7 +75,7 @@ def test_integer_exact_and_writes_only_c(gpu, shape, out):
 def test_repeatable(gpu):
     """Two calls in a row (the second reuses the library workspace and version
     10's counters): bitwise equal."""
-    A, B = make_inputs(1000, 1001, 4001, "normal", seed=11)
+    A, B = make_inputs(300, 201, 4095, "normal", seed=11)
     C1 = run_gemm(15, A, B, "f16")
     C2 = run_gemm(15, A, B, "f16")
     assert np.array_equal(C1.view(np.uint16), C2.view(np.uint16))

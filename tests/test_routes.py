@@ -81,6 +81,10 @@ def test_odd_k_of_few_rows(kernel, call, name):
     ((F16, 15, 300, 50001, 129), "f16_pp16"),
     ((F16, 15, 4096, 8192, 255), "f16_pp16"),
     ((F16, 15, 2049, 2051, 2052), "f16_pp16"),     # past 2^33
+    ((F16, 15, 129, 9, 4097), "f16_pp16_sk"),
+    ((F16, 15, 300, 201, 4095), "f16_pp16_sk"),
+    ((F16, 15, 4000, 4001, 33), "f16_pp16_edge"),
+    ((F16, 15, 4096, 4095, 1032), "f16_pp16_edge"),
 ])
 def test_copies_of_version_15(kernel, call, name):
     assert name in kernel(*call)
