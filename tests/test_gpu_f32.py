@@ -27,9 +27,8 @@ from gpu_util import announce, make_inputs
 
 pytestmark = pytest.mark.gpu
 
-# version 1 on 256 CUs: 64 x 64 tiles for every shape here but the last two
-# (the bounds-checked 128 x 256 kernel at 4000 x 4000, the asm kernel at
-# 4096 x 4096)
+# version 1 on 256 CUs: the matrix cores for every shape here but the last (the
+# asm kernel at 4096 x 4096)
 SHAPES_V1 = [(128, 128, 16), (256, 384, 64), (512, 512, 512), (1, 1, 1), (17, 33, 65), (130, 250, 70),
              (128, 256, 16), (256, 512, 32), (384, 768, 48), (1024, 512, 1024), (128, 256, 2000),
              (4000, 4000, 40), (4096, 4096, 32)]

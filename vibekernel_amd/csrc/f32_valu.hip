@@ -30,7 +30,6 @@ constexpr int kTM = 128;             // tile rows
 constexpr int kCG = 4;               // 64-column groups per tile
 constexpr int kTN = 64 * kCG;        // tile columns
 constexpr int kBK = 16;
-constexpr int kApitch = kTM + 4;     // As_t[k][m] row pitch (floats)
 
 // Every VGPR from v32 up: the registers the asm kernel below uses itself.
 #define VK_CLOBBER_V32_V255 \
@@ -86,14 +85,13 @@ bool asm_offsets_fit(size_t m, size_t n, size_t k) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 // Full tiles (M % 128, N % 256, K % 16 == 0, 16-byte aligned operands): the
-// same tile, thread mapping and summation order as the kernel above, with
-// the k-loop written as one asm block so that the registers are chosen here
-// rather than by the compiler, and the k-tiles staged by direct-to-LDS loads.
+// k-loop is one asm block so that the registers are chosen here rather than by
+// the compiler, and the k-tiles are staged by direct-to-LDS loads.
 //
 // Registers.  A v_fmac_f32 whose three operands (accumulator, a, b) sit in
 // the same VGPR bank (register number mod 4) issues at half rate; with two in
 // one bank there is no measurable loss (microbenchmarks on MI355X: 63-70
-// against 124-139 TFLOP/s).  For the C++ kernel the compiler put every
+// against 124-139 TFLOP/s).  In a C++ form of the loop the compiler put every
 // accumulator in its b operand's bank, and a quarter of the 256 FMAs of a
 // k-step pair also had a in that bank.  Here:
 //   acc[i][j]  v[128 + 16 i + ((j + 1) % 16)]   bank (j + 1) % 4
@@ -118,7 +116,7 @@ bool asm_offsets_fit(size_t m, size_t n, size_t k) {
 // 1296.5 us against 1310.4 us for the same k-loop staged through registers
 // with A transposed by 4-byte LDS stores (106.0 against 104.9 TFLOP/s).
 // Each output is one v_fmac_f32 per k in ascending order from 0: the same
-// sums, bit for bit, as the C++ kernel and the oracle.  C is stored with sc1
+// sums, bit for bit, as f32_any.hip's and the oracle's.  C is stored with sc1
 // (written through the XCD's L2, not left dirty for the end-of-kernel
 // write-back): 1302.5 against 1314.6 us per launch at 4096^3 (3 interleaved
 // rounds on one box).
@@ -330,8 +328,8 @@ void register_f32_valu() {
   e.version = 1;
   e.in_dtype = VK_DTYPE_F32;
   e.name = "f32_v1_valu";
-  e.caps = make_caps(1, VK_DTYPE_F32, kOutF32, 1, 1, 1, 4, kTM, kTN, kBK, 256,
-                     2 * kBK * (kApitch + kTN) * 4, 0, 0);
+  // the asm kernel's tile, threads and LDS (f32_any.hip's: 512 threads, up to 80 KB)
+  e.caps = make_caps(1, VK_DTYPE_F32, kOutF32, 1, 1, 1, 4, kTM, kTN, kBK, 256, 2 * kBK * (kTM + kTN) * 4, 0, 0);
   e.launch = launch_f32;
   e.workspace = nullptr;
   e.shape_ok = f32_shape_ok;
