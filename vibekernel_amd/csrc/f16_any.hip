@@ -144,7 +144,8 @@ __global__ __launch_bounds__(kThreads, 2) void f16_any_kernel(const half_t* __re
     return __builtin_bit_cast(uint4v, back == 8 ? (unsigned __int128)0 : x >> (16 * back));
   };
   auto load_elements = [&](const half_t* p, int64_t valid, const half_t* safe) {
-    half8 h;
+    half8 h = {};
+    if (valid <= 0) return __builtin_bit_cast(uint4v, h);  // most chunks, K or N below 8
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       const half_t x = (e < valid ? p + e : safe)[0];
@@ -223,6 +224,7 @@ __global__ __launch_bounds__(kThreads, 2) void f16_any_kernel(const half_t* __re
     read(f[0], buf, 0);
 #pragma unroll
     for (int h = 0; h < BK / 64; h++) {
+      if (kNarrow && h > 0 && K <= 64 * h) break;
       if (h + 1 < BK / 64) read(f[(h + 1) & 1], buf, h + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
