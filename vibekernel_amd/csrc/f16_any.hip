@@ -16,7 +16,9 @@
 //    not stored); one that N cuts short reads on into the next row, which
 //    exists except at the end of B: in the last k-tile the chunks that K or N
 //    cuts are loaded from 8 elements further back at most and shifted, zeros
-//    past the edge in both operands (N or K below 8: element by element).
+//    past the edge in both operands (N or K below 8: element by element);
+//  * C goes straight from the registers, 32 bytes of a row at a time, or through
+//    LDS in whole rows of a wave's block (launch_nb's rule).
 // Measured (us per launch, fresh operands): version 1 before, whose 128 x 128
 // tiles loaded element by element, 64 x 62 x 65 12.2, now 4.5; 100 x 300 x 70
 // 15.9 / 5.5; 300 x 200 x 4095 950 / 28.7; 700 x 8191 x 2048 474 / 64.  A k-tile
