@@ -106,13 +106,16 @@ def test_small_k_of_fp32_version_1(kernel, call, name):
     assert name in kernel(*call)
 
 
-# few rows of fp32 version 3: small whole k-tiles keep the tiles
+# few rows of fp32 version 3: small whole k-tiles, and a second round of column blocks from 33 rows, keep the tiles
 @pytest.mark.parametrize("call,name", [
     ((F32, 3, 32, 16384, 64), "f32_mfma4"), ((F32, 3, 32, 16384, 80), "f32_stream"),
     ((F32, 3, 32, 16384, 128), "f32_stream"), ((F32, 3, 32, 20000, 96), "f32_mfma4"),
     ((F32, 3, 32, 32768, 64), "f32_stream"), ((F32, 3, 16, 16384, 64), "f32_mfma4"),
     ((F32, 3, 16, 20000, 64), "f32_stream"), ((F32, 3, 64, 262144, 64), "f32_mfma4"),
     ((F32, 3, 64, 262144, 96), "f32_stream"), ((F32, 3, 48, 262144, 64), "f32_stream"),
+    ((F32, 3, 64, 16384, 4096), "f32_stream"), ((F32, 3, 64, 16388, 4096), "f32_mfma4"),
+    ((F32, 3, 33, 32640, 1024), "f32_mfma4"), ((F32, 3, 33, 32644, 1024), "f32_stream"),
+    ((F32, 3, 32, 20000, 4096), "f32_stream"),
 ])
 def test_few_rows_of_fp32_version_3(kernel, call, name):
     assert name in kernel(*call)

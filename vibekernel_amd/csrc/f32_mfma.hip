@@ -896,7 +896,7 @@ bool f32_mfma_shape_ok(size_t m, size_t n, size_t k) {
 // offsets).
 // Few rows: f32_stream.hip, within the workspace of the tiles' split.
 hipError_t launch_f32_mfma_edge(const GemmArgs& a) {
-  if (f32_stream_takes(a.m, a.n, a.k)) return f32_stream_launch(a, f32_workspace(a.m, a.n, a.k, a.num_cus));
+  if (f32_stream_takes(a.m, a.n, a.k, a.num_cus)) return f32_stream_launch(a, f32_workspace(a.m, a.n, a.k, a.num_cus));
   if (f32_small_tiles(a.m, a.n, a.num_cus)) return launch_f32_small<true>(a);
   return a.k % 32 == 0 ? launch_w4<4, true, false>(a, SkPlan{0, 0, 1, 1}) : launch_bk<32, true>(a);
 }
@@ -905,7 +905,7 @@ hipError_t launch_f32_mfma_edge(const GemmArgs& a) {
 // zero; few rows whose K is not split leave the workspace as it was.
 int f32_edge_workspace_kind(size_t m, size_t n, size_t k, int num_cus) {
   const bool unsplit =
-      f32_stream_takes(m, n, k) && f32_stream_pieces(m, n, k, f32_workspace(m, n, k, num_cus), num_cus) == 1;
+      f32_stream_takes(m, n, k, num_cus) && f32_stream_pieces(m, n, k, f32_workspace(m, n, k, num_cus), num_cus) == 1;
   return unsplit ? kWorkspaceUntouched : 0;
 }
 

@@ -177,15 +177,22 @@ hipError_t launch_mb(const GemmArgs& a, size_t ws_limit) {
 // 4096 x 4096 / 8192 x 8192 13.4 / 21.1 / 28.5 / 79 against 10.8 / 17.6 / 31.7 /
 // 98.8.  What bounds the large ones is the read of B (16 x 8192 x 8192: 5.0
 // TB/s), the small ones the launch and the pieces' hand-off.
+// More than 32 rows are bound by the matrix cores, where a second column block on
+// some of the CUs takes as long as one on all of them.  The 64 x 64 tiles (fewer
+// 128 x 128 ones than CUs) do better there, and keep it: 56 x 18000 x 4096 205 us
+// against 105, 64 x 21776 x 1572 83.6 / 49.3, 64 x 28000 x 512 28.0 / 20.7, 48 x
+// 32000 x 2048 81 / 71; from the 128 x 128 tiles on they do not (48 x 32704 x 2048
+// 82 / 128, 56 x 34000 x 512 36 / 64, 64 x 40000 x 4096 302 / 314).
 // Where K is one to three of the tiles' whole 32-deep k-tiles, the waves have a
 // step or two each and their sum is most of the time, so the tiles keep a grid of
 // up to one column block per CU (two from 17 rows) and, for 64 rows, the largest
 // ones: 32 x 16384 x 64 / 96 4.8 / 5.5 us against 4.4 / 4.9, 32 x 20000 x 64 6.8 /
 // 5.5, 64 x 262144 x 64 56.3 / 51.6; but 16 x 20000 x 96 6.2 / 6.4, 32 x 32768 x 64
 // 7.3 / 9.0, 64 x 262144 x 128 72 / 79.
-bool f32_stream_takes(size_t m, size_t n, size_t k) {
-  if (m > 32 && n * k < ((size_t)1 << 23)) return false;
-  if (k % 32 == 0 && m <= 32 && k <= 96 && n <= (m <= 16 ? 16384 : 32767)) return false;
+bool f32_stream_takes(size_t m, size_t n, size_t k, int num_cus) {
+  const size_t c = num_cus > 0 ? num_cus : 1, blocks = (n + kNC - 1) / kNC;
+  if (m > 32 && (n * k < ((size_t)1 << 23) || (blocks > c && (n + 127) / 128 < c))) return false;
+  if (k % 32 == 0 && m <= 32 && k <= 96 && (blocks <= c || (m > 16 && blocks < 2 * c))) return false;
   if (k % 32 == 0 && m > 56 && k <= 64) return false;
   return m >= 1 && m <= kMaxRows && n >= 4 && n % 4 == 0 && n < (1u << 25) && k >= 4 && k % 4 == 0 && k < (1u << 23);
 }

@@ -68,7 +68,7 @@ hipError_t f32_any_launch(const GemmArgs& a);
 // fp32, few rows, N and K multiples of 4 (f32_stream.hip), with at most
 // ws_limit bytes of the workspace: none where _pieces, the workgroups per
 // column block, is 1.
-bool f32_stream_takes(size_t m, size_t n, size_t k);
+bool f32_stream_takes(size_t m, size_t n, size_t k, int num_cus);
 int f32_stream_pieces(size_t m, size_t n, size_t k, size_t ws_limit, int num_cus);
 hipError_t f32_stream_launch(const GemmArgs& a, size_t ws_limit);
 
