@@ -66,8 +66,10 @@ def test_odd_k_of_few_rows(kernel, call, name):
 # version 15 through registers or through copies and version 10
 @pytest.mark.parametrize("call,name", [
     ((F16, 15, 1000, 1001, 999), "f16_any"),
-    ((F16, 15, 700, 700, 10239), "f16_any"),       # few tiles: K up to 10240
-    ((F16, 15, 700, 700, 10241), "f16_pp16"),
+    ((F16, 15, 700, 700, 11263), "f16_any"),       # few tiles: odd K up to 11264
+    ((F16, 15, 700, 700, 11265), "f16_pp16"),
+    ((F16, 15, 700, 700, 14332), "f16_any"),       # even K up to 14336
+    ((F16, 15, 700, 700, 14338), "f16_pp16"),
     ((F16, 15, 300, 200, 1023), "f16_any"),        # fewer still: K up to 1024
     ((F16, 15, 300, 200, 4095), "f16_pp16"),
     ((F16, 15, 128, 50001, 1023), "f16_any"),      # half-empty 256 x 256 tiles

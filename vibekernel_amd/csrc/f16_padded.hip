@@ -125,10 +125,12 @@ bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_str
 // multiply-adds.  us per launch, f16_any.hip / copies and version 10:
 //  * while 64 x 64 tiles are at most 4 per CU (f16_any_launch's rule for them): 1000
 //    x 1001 x 1023 13.0 / 34.3, 2000 x 2001 x 2001 48 / 55; but a workgroup's
-//    k-loop is one chain, which the copies' split sum cuts in 8: 700 x 700 x 8191
-//    49.6 / 61, x 12287 77 / 79, x 16383 105 / 90 (200 x 500 x 32767 215 against
-//    129), and a few tiles of K > 1024 are slower from the start (300 x 200 x
-//    4095 28.7 / 49 with 20 tiles of 4095, 160 CUs idle);
+//    k-loop is one chain, which the copies' split sum cuts in 8: 224 x 968 x 10242
+//    48 / 64, x 14340 70 / 75, x 16380 85 / 80; odd K, whose rows of A straddle dwords,
+//    224 x 968 x 10241 64 / 64, 700 x 700 x 11267 66 / 72, 1000 x 136 x 11267 68 / 66,
+//    200 x 500 x 32767 215 / 129.  Fewer tiles than an eighth of the CUs keep version
+//    10's split sum (and its bits) from K = 1025 on, though 300 x 200 x 4095 takes 28.7
+//    / 49;
 //  * where half of each 256 x 256 tile is empty: 128 x 50001 x 1023 53 / 67, 100000
 //    x 65 x 513 63 / 79;
 //  * while 128 x 128 tiles are at most 2 per CU, up to K = 1024: 1000 x 8001 x 129
@@ -146,7 +148,7 @@ bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
   if (m * n * k > (size_t)1 << 33) return false;
   const size_t c = num_cus;
   auto tiles = [&](size_t t) { return (m + t - 1) / t * ((n + t - 1) / t); };
-  if (tiles(64) <= 4 * c) return k <= 1024 || (8 * tiles(64) >= c && k <= 10240);
+  if (tiles(64) <= 4 * c) return k <= 1024 || (8 * tiles(64) >= c && k <= (k % 2 ? 11264 : 14336));
   if (m <= 128 || n <= 128) return true;
   if (tiles(128) <= 2 * c) return k <= 1024;
   const size_t filled = 100 * m * n / (tiles(256) * 65536);  // per cent of the 256 x 256 tiles
