@@ -70,6 +70,8 @@ def test_odd_k_of_few_rows(kernel, call, name):
     ((F16, 15, 700, 700, 11265), "f16_pp16"),
     ((F16, 15, 700, 700, 14332), "f16_any"),       # even K up to 14336
     ((F16, 15, 700, 700, 14338), "f16_pp16"),
+    ((F16, 15, 700, 701, 12288), "f16_any"),       # K a multiple of 8 up to 12288
+    ((F16, 15, 700, 701, 12296), "f16_pp16"),
     ((F16, 15, 300, 200, 1023), "f16_any"),        # fewer still: K up to 1024
     ((F16, 15, 300, 200, 4095), "f16_pp16"),
     ((F16, 15, 128, 50001, 1023), "f16_any"),      # half-empty 256 x 256 tiles

@@ -128,7 +128,8 @@ bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_str
 //    k-loop is one chain, which the copies' split sum cuts in 8: 224 x 968 x 10242
 //    48 / 64, x 14340 70 / 75, x 16380 85 / 80; odd K, whose rows of A straddle dwords,
 //    224 x 968 x 10241 64 / 64, 700 x 700 x 11267 66 / 72, 1000 x 136 x 11267 68 / 66,
-//    200 x 500 x 32767 215 / 129.  Fewer tiles than an eighth of the CUs keep version
+//    200 x 500 x 32767 215 / 129; K a multiple of 8, where only B is copied, 1984 x 116 x
+//    12288 68 / 63, x 14336 78 / 66, 224 x 969 x 12288 61 / 68, x 14336 75 / 72.  Fewer tiles than an eighth of the CUs keep version
 //    10's split sum (and its bits) from K = 1025 on, though 300 x 200 x 4095 takes 28.7
 //    / 49;
 //  * where half of each 256 x 256 tile is empty: 128 x 50001 x 1023 53 / 67, 100000
@@ -148,7 +149,7 @@ bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
   if (m * n * k > (size_t)1 << 33) return false;
   const size_t c = num_cus;
   auto tiles = [&](size_t t) { return (m + t - 1) / t * ((n + t - 1) / t); };
-  if (tiles(64) <= 4 * c) return k <= 1024 || (8 * tiles(64) >= c && k <= (k % 2 ? 11264 : 14336));
+  if (tiles(64) <= 4 * c) return k <= 1024 || (8 * tiles(64) >= c && k <= (k % 2 ? 11264 : k % 8 ? 14336 : 12288));
   if (m <= 128 || n <= 128) return true;
   if (tiles(128) <= 2 * c) return k <= 1024;
   const size_t filled = 100 * m * n / (tiles(256) * 65536);  // per cent of the 256 x 256 tiles
