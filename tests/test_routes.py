@@ -74,8 +74,20 @@ def test_odd_k_of_few_rows(kernel, call, name):
     ((F16, 15, 700, 701, 12296), "f16_pp16"),
     ((F16, 15, 300, 200, 1023), "f16_any"),        # fewer still: K up to 1024
     ((F16, 15, 300, 200, 4095), "f16_pp16"),
+    ((F16, 15, 1000, 2001, 4096), "f16_any"),      # more tiles than CUs
+    ((F16, 15, 10000, 101, 6144), "f16_pp16"),
+    ((F16, 15, 8000, 257, 2048), "f16_any"),       # two per CU
+    ((F16, 15, 8000, 257, 3072), "f16_pp16"),
     ((F16, 15, 128, 50001, 1023), "f16_any"),      # half-empty 256 x 256 tiles
     ((F16, 15, 100000, 65, 513), "f16_any"),
+    ((F16, 15, 100000, 65, 512), "f16_pp16"),
+    ((F16, 15, 46840, 1, 688), "f16_pp16"),        # N below 8
+    ((F16, 15, 46840, 1, 191), "f16_any"),
+    ((F16, 15, 100000, 7, 104), "f16_pp16"),
+    ((F16, 15, 2000, 1, 688), "f16_any"),
+    ((F16, 15, 16000, 401, 512), "f16_pp16"),      # only B copied
+    ((F16, 15, 50000, 305, 64), "f16_pp16"),
+    ((F16, 15, 300, 50001, 130), "f16_any"),
     ((F16, 15, 1000, 8001, 1023), "f16_any"),      # two 128 x 128 tiles per CU
     ((F16, 15, 1500, 3001, 1801), "f16_pp16"),
     ((F16, 15, 50000, 304, 191), "f16_any"),       # few columns

@@ -122,25 +122,31 @@ hipError_t repitch(const void* src, void* dst, size_t rows, size_t width, size_t
 bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_stream_takes(m, n, k); }
 
 // Neither do products that cannot earn the copies back (f16_any.hip), up to 2^33
-// multiply-adds.  us per launch, f16_any.hip / copies and version 10:
+// multiply-adds.  Where K is a multiple of 8 only B is copied, and the copies earn
+// more.  us per launch, f16_any.hip / copies and version 10:
+//  * N below 8, whose B is loaded element by element: 100000 x 7 x 130 30 / 40, x 64
+//    16.4 / 19.0, x 128 27 / 22, 46840 x 1 x 688 75 / 26, 2000 x 1 x 1024 33 / 26;
 //  * while 64 x 64 tiles are at most 4 per CU (f16_any_launch's rule for them): 1000
 //    x 1001 x 1023 13.0 / 34.3, 2000 x 2001 x 2001 48 / 55; but a workgroup's
 //    k-loop is one chain, which the copies' split sum cuts in 8: 224 x 968 x 10242
 //    48 / 64, x 14340 70 / 75, x 16380 85 / 80; odd K, whose rows of A straddle dwords,
 //    224 x 968 x 10241 64 / 64, 700 x 700 x 11267 66 / 72, 1000 x 136 x 11267 68 / 66,
-//    200 x 500 x 32767 215 / 129; K a multiple of 8, where only B is copied, 1984 x 116 x
-//    12288 68 / 63, x 14336 78 / 66, 224 x 969 x 12288 61 / 68, x 14336 75 / 72.  Fewer tiles than an eighth of the CUs keep version
-//    10's split sum (and its bits) from K = 1025 on, though 300 x 200 x 4095 takes 28.7
-//    / 49;
+//    200 x 500 x 32767 215 / 129; B alone copied, 224 x 969 x 12288 61 / 68, x 14336 75
+//    / 72, with more tiles than CUs 10000 x 101 x 4096 48 / 46, 1000 x 2001 x 4096 40 /
+//    48, with two per CU 8000 x 257 x 2048 36 / 45, x 3072 51 / 43.  Fewer tiles than an
+//    eighth of the CUs keep version 10's split sum (and its bits) from K = 1025 on,
+//    though 300 x 200 x 4095 takes 28.7 / 49;
 //  * where half of each 256 x 256 tile is empty: 128 x 50001 x 1023 53 / 67, 100000
-//    x 65 x 513 63 / 79;
+//    x 65 x 513 63 / 79, but 100000 x 65 x 512 56 / 42, x 256 35 / 31;
 //  * while 128 x 128 tiles are at most 2 per CU, up to K = 1024: 1000 x 8001 x 129
-//    18.4 / 20.4, 3000 x 1500 x 1023 35 / 40, 1500 x 3001 x 1801 63 / 52;
+//    18.4 / 20.4, 3000 x 1500 x 1023 35 / 40, 1500 x 3001 x 1801 63 / 52, 16000 x 401 x
+//    512 24.7 / 20.2;
 //  * past that few columns up to K = 256, whose copy of A is most of the work:
 //    50000 x 304 x 193 32 / 36, x 257 47 / 43, 50000 x 200 x 193 24 / 29, x 385 45 /
-//    39, 30000 x 600 x 129 28.0 / 29.6; 50000 x 400 x 65 28.7 / 26.3; and few rows of whole 8-column chunks: 300 x
-//    50000 x 193 32 / 35, x 257 47 / 40; 300 x 50001 x 65 30.3 / 29.5, 400 x 50000 x
-//    65 31.5 / 26.3, 129 x 100000 x 129 38.7 / 34.0;
+//    39, 30000 x 600 x 129 28.0 / 29.6; 50000 x 400 x 65 28.7 / 26.3; and few rows whose
+//    A or B starts on dwords: 300 x 50000 x 193 32 / 35, x 257 47 / 40; 300 x 50001 x 65
+//    30.3 / 29.5, x 130 28.6 / 31.8; 400 x 50000 x 65 31.5 / 26.3, 129 x 100000 x 129
+//    38.7 / 34.0;
 //  * the rest take the copies: 4000 x 4000 x 33 18.6 / 15.3, 4096 x 8192 x 255 55 /
 //    40, 8192 x 8193 x 65 111 / 59.
 bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
@@ -148,14 +154,21 @@ bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
   if ((m + 127) / 128 > 65535) return false;            // rows of its tiles are grid.y
   if (m * n * k > (size_t)1 << 33) return false;
   const size_t c = num_cus;
+  const bool copy_a = k % 8 != 0;
   auto tiles = [&](size_t t) { return (m + t - 1) / t * ((n + t - 1) / t); };
-  if (tiles(64) <= 4 * c) return k <= 1024 || (8 * tiles(64) >= c && k <= (k % 2 ? 11264 : k % 8 ? 14336 : 12288));
-  if (m <= 128 || n <= 128) return true;
-  if (tiles(128) <= 2 * c) return k <= 1024;
+  const size_t small = tiles(64);
+  if (n < 8) return k <= (copy_a ? 192 : 96) || (k <= 768 && m * k < (size_t)3 << 19);
+  if (small <= 4 * c) {
+    const size_t deepest = k % 2 ? 11264 : copy_a ? 14336 : small <= c ? 12288 : small <= 2 * c ? 4608 : 2560;
+    return k <= 1024 || (8 * small >= c && k <= deepest);
+  }
+  if (m <= 128) return true;
+  if (n <= 128) return copy_a || k < 256;
+  if (tiles(128) <= 2 * c) return k <= (copy_a ? 1024 : 256);
+  if (!copy_a || k > 256) return false;
   const size_t filled = 100 * m * n / (tiles(256) * 65536);  // per cent of the 256 x 256 tiles
   const bool few = tiles(128) <= 5 * c;
-  if (k > 256) return false;
-  return m > n ? n <= 256 || filled <= (few ? 80 : 60) : n % 8 == 0 && k > 64 && filled <= 60 && few;
+  return m > n ? n <= 256 || filled <= (few ? 80 : 60) : (n % 8 == 0 || k % 2 == 0) && k > 64 && filled <= 60 && few;
 }
 
 hipError_t launch_padded(const GemmArgs& a) {
