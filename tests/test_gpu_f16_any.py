@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 # from (1990, 2047, 33) on: 128 x 128 tiles (256 CUs)
 SHAPES = [(1, 1, 1), (2, 7, 9), (5, 9, 7), (63, 65, 128), (64, 64, 127), (65, 63, 129), (1, 129, 255), (129, 12, 257),
           (200, 130, 640), (64, 67, 512), (100, 300, 70), (1990, 2047, 33), (2047, 1985, 130), (1601, 1600, 191),
-          (1600, 1609, 320), (25000, 5, 65), (25000, 70, 6)]
+          (1600, 1609, 320), (25000, 5, 65), (25000, 70, 6), (200, 7, 300), (65, 1, 129),
+          (64, 5, 256), (130, 3, 1023), (67000, 7, 200)]
 
 
 def _run(A, B, out, shift):
@@ -61,7 +62,7 @@ def test_rows_of_c(gpu, oracle, shape, shift):
     assert np.array_equal(_run(A, B, "f16", shift).astype(np.float32), A.astype(np.float32) @ B.astype(np.float32))
 
 
-@pytest.mark.parametrize("shape", [(3, 5, 35), (70, 67, 130), (1700, 1603, 260)])
+@pytest.mark.parametrize("shape", [(3, 5, 35), (70, 67, 130), (1700, 1603, 260), (70, 5, 200), (70, 67, 5)])
 def test_values_past_the_edges_never_reach_c(gpu, shape):
     """A[1][0] is what row 0 reads past K, B[k-1][0] what row k-2 reads past
     N: infinite, they may only reach row 1 and column 0."""

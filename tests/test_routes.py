@@ -82,9 +82,11 @@ def test_odd_k_of_few_rows(kernel, call, name):
     ((F16, 15, 100000, 65, 513), "f16_any"),
     ((F16, 15, 100000, 65, 512), "f16_pp16"),
     ((F16, 15, 46840, 1, 688), "f16_pp16"),        # N below 8
-    ((F16, 15, 46840, 1, 191), "f16_any"),
-    ((F16, 15, 100000, 7, 104), "f16_pp16"),
+    ((F16, 15, 46840, 1, 383), "f16_any"),
+    ((F16, 15, 100000, 7, 128), "f16_pp16"),
+    ((F16, 15, 100000, 7, 120), "f16_any"),
     ((F16, 15, 2000, 1, 688), "f16_any"),
+    ((F16, 15, 2000, 1, 776), "f16_pp16"),
     ((F16, 15, 16000, 401, 512), "f16_pp16"),      # only B copied
     ((F16, 15, 50000, 305, 64), "f16_pp16"),
     ((F16, 15, 300, 50001, 130), "f16_any"),

@@ -16,7 +16,8 @@
 //    not stored); one that N cuts short reads on into the next row, which
 //    exists except at the end of B: in the last k-tile the chunks that K or N
 //    cuts are loaded from 8 elements further back at most and shifted, zeros
-//    past the edge in both operands (N or K below 8: element by element);
+//    past the edge in both operands (an operand whose rows are shorter than 8:
+//    element by element);
 //  * C goes straight from the registers, 32 bytes of a row at a time, or through
 //    LDS in whole rows of a wave's block (launch_nb's rule).
 // Measured (us per launch, fresh operands): version 1 before, whose 128 x 128
@@ -165,8 +166,9 @@ __global__ __launch_bounds__(kThreads, 2) void f16_any_kernel(const half_t* __re
     for (int i = 0; i < L; i++) {
       const int64_t va = left - ak[i], vb = bk[i] < left ? N - bc[i] : 0;
       if constexpr (kNarrow) {
-        r.a[i] = load_elements(pa[i] + t * BK, va, A);
-        r.b[i] = load_elements(pb[i] + t * BK * N, vb, B);
+        const half_t *a = pa[i] + t * BK, *b = pb[i] + t * BK * N;
+        r.a[i] = K < 8 ? load_elements(a, va, A) : load_cut(a, va, A);
+        r.b[i] = N < 8 ? load_elements(b, vb, B) : load_cut(b, vb, B);
       } else {
         r.a[i] = load_cut(pa[i] + t * BK, va, A);
         r.b[i] = load_cut(pb[i] + t * BK * N, vb, B);

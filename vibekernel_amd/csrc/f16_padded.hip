@@ -124,8 +124,9 @@ bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_str
 // Neither do products that cannot earn the copies back (f16_any.hip), up to 2^33
 // multiply-adds.  Where K is a multiple of 8 only B is copied, and the copies earn
 // more.  us per launch, f16_any.hip / copies and version 10:
-//  * N below 8, whose B is loaded element by element: 100000 x 7 x 130 30 / 40, x 64
-//    16.4 / 19.0, x 128 27 / 22, 46840 x 1 x 688 75 / 26, 2000 x 1 x 1024 33 / 26;
+//  * N below 8, whose B is loaded element by element: 100000 x 7 x 258 51 / 57, x 1025
+//    182 / 140, x 96 16.5 / 22, 300000 x 2 x 128 59 / 48, 46840 x 1 x 688 60 / 26; 20000 x
+//    3 x 256 9.8 / 13.8, 2000 x 1 x 688 16.8 / 20.7, x 1024 26.4 / 25.9;
 //  * while 64 x 64 tiles are at most 4 per CU (f16_any_launch's rule for them): 1000
 //    x 1001 x 1023 13.0 / 34.3, 2000 x 2001 x 2001 48 / 55; but a workgroup's
 //    k-loop is one chain, which the copies' split sum cuts in 8: 224 x 968 x 10242
@@ -157,7 +158,7 @@ bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
   const bool copy_a = k % 8 != 0;
   auto tiles = [&](size_t t) { return (m + t - 1) / t * ((n + t - 1) / t); };
   const size_t small = tiles(64);
-  if (n < 8) return k <= (copy_a ? 192 : 96) || (k <= 768 && m * k < (size_t)3 << 19);
+  if (n < 8) return k <= (copy_a ? 384 : 120) || (k <= 768 && m * k < (size_t)1 << 23);
   if (small <= 4 * c) {
     const size_t deepest = k % 2 ? 11264 : copy_a ? 14336 : small <= c ? 12288 : small <= 2 * c ? 4608 : 2560;
     return k <= 1024 || (8 * small >= c && k <= deepest);
