@@ -88,6 +88,11 @@ def test_odd_k_of_few_rows(kernel, call, name):
     ((F16, 15, 2000, 1, 688), "f16_any"),
     ((F16, 15, 2000, 1, 776), "f16_pp16"),
     ((F16, 15, 16000, 401, 512), "f16_pp16"),      # only B copied
+    ((F16, 15, 236, 16964, 1024), "f16_any"),      # and its rows start on dwords
+    ((F16, 15, 512, 4978, 3368), "f16_any"),
+    ((F16, 15, 512, 4979, 2568), "f16_pp16"),
+    ((F16, 15, 3000, 1500, 1500), "f16_any"),      # even K
+    ((F16, 15, 3000, 1500, 1025), "f16_pp16"),
     ((F16, 15, 50000, 305, 64), "f16_pp16"),
     ((F16, 15, 300, 50001, 130), "f16_any"),
     ((F16, 15, 1000, 8001, 1023), "f16_any"),      # two 128 x 128 tiles per CU

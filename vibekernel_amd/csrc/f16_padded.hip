@@ -134,14 +134,16 @@ bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_str
 //    224 x 968 x 10241 64 / 64, 700 x 700 x 11267 66 / 72, 1000 x 136 x 11267 68 / 66,
 //    200 x 500 x 32767 215 / 129; B alone copied, 224 x 969 x 12288 61 / 68, x 14336 75
 //    / 72, with more tiles than CUs 10000 x 101 x 4096 48 / 46, 1000 x 2001 x 4096 40 /
-//    48, with two per CU 8000 x 257 x 2048 36 / 45, x 3072 51 / 43.  Fewer tiles than an
+//    48, with two per CU 8000 x 257 x 2048 36 / 45, x 3072 51 / 43, 512 x 4978 x 2624 38
+//    / 47.  Fewer tiles than an
 //    eighth of the CUs keep version 10's split sum (and its bits) from K = 1025 on,
 //    though 300 x 200 x 4095 takes 28.7 / 49;
 //  * where half of each 256 x 256 tile is empty: 128 x 50001 x 1023 53 / 67, 100000
 //    x 65 x 513 63 / 79, but 100000 x 65 x 512 56 / 42, x 256 35 / 31;
-//  * while 128 x 128 tiles are at most 2 per CU, up to K = 1024: 1000 x 8001 x 129
-//    18.4 / 20.4, 3000 x 1500 x 1023 35 / 40, 1500 x 3001 x 1801 63 / 52, 16000 x 401 x
-//    512 24.7 / 20.2;
+//  * while 128 x 128 tiles are at most 2 per CU, up to K = 1024, or 1536 even: 1000 x
+//    8001 x 129 18.4 / 20.4, 3000 x 1500 x 1023 35 / 40, x 1500 43 / 46, 1500 x 3001 x
+//    1801 63 / 52; B alone copied, 16000 x 401 x 512 24.7 / 20.2, 236 x 16964 x 1024 36
+//    / 43;
 //  * past that few columns up to K = 256, whose copy of A is most of the work:
 //    50000 x 304 x 193 32 / 36, x 257 47 / 43, 50000 x 200 x 193 24 / 29, x 385 45 /
 //    39, 30000 x 600 x 129 28.0 / 29.6; 50000 x 400 x 65 28.7 / 26.3; and few rows whose
@@ -160,12 +162,13 @@ bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
   const size_t small = tiles(64);
   if (n < 8) return k <= (copy_a ? 384 : 120) || (k <= 768 && m * k < (size_t)1 << 23);
   if (small <= 4 * c) {
-    const size_t deepest = k % 2 ? 11264 : copy_a ? 14336 : small <= c ? 12288 : small <= 2 * c ? 4608 : 2560;
+    size_t deepest = k % 2 ? 11264 : copy_a ? 14336 : small <= c ? 12288 : small <= 2 * c ? 4608 : 2560;
+    if (n % 2 == 0 && !copy_a && small > c) deepest += 1536;  // B's rows start on dwords
     return k <= 1024 || (8 * small >= c && k <= deepest);
   }
   if (m <= 128) return true;
   if (n <= 128) return copy_a || k < 256;
-  if (tiles(128) <= 2 * c) return k <= (copy_a ? 1024 : 256);
+  if (tiles(128) <= 2 * c) return k <= (!copy_a && n % 2 ? 256 : k % 2 ? 1024 : 1536);
   if (!copy_a || k > 256) return false;
   const size_t filled = 100 * m * n / (tiles(256) * 65536);  // per cent of the 256 x 256 tiles
   const bool few = tiles(128) <= 5 * c;
