@@ -154,19 +154,20 @@ __global__ __launch_bounds__(kThreads, NB == 1 ? 4 : 2) void f32_any_kernel(cons
   auto valid_b = [&](int i, int64_t t) { return bk[i] < K - t * BK ? N - bc[i] : 0; };
   auto load = [&](Chunks& r, int64_t t) {
     if constexpr (kTiles == 0) {
-      if (!narrow && (t < nk - 1 || (K % BK == 0 && N % 4 == 0))) {
+      if (narrow || (t == nk - 1 && (K % BK != 0 || N % 4 != 0))) {
+        const int64_t left = K - t * BK;  // k of this k-tile
+#pragma unroll
+        for (int i = 0; i < L; i++)
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const bool in_a = ak[i] + q < left, in_b = bk[i] < left && bc[i] + q < N;
+            const float va = (in_a ? pa[i] + t * BK + q : A)[0], vb = (in_b ? pb[i] + t * BK * N + q : B)[0];
+            r.a[i][q] = in_a ? va : 0.0f;
+            r.b[i][q] = in_b ? vb : 0.0f;
+          }
+      } else {
         load_whole(r, t);
-        return;
       }
-#pragma unroll
-      for (int i = 0; i < L; i++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const bool in_a = q < valid_a(i, t), in_b = q < valid_b(i, t);
-          const float va = (in_a ? pa[i] + t * BK + q : A)[0], vb = (in_b ? pb[i] + t * BK * N + q : B)[0];
-          r.a[i][q] = in_a ? va : 0.0f;
-          r.b[i][q] = in_b ? vb : 0.0f;
-        }
       return;
     }
     const bool ca = cut_a(t), cb = cut_b(t);
