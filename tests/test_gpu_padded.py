@@ -21,7 +21,7 @@ SHAPES = [(1000, 1001, 1000), (999, 1000, 1001), (17, 33, 65), (1, 1, 1), (257, 
           (300, 200, 4095), (1024, 1024, 1023)]
 # through the copies, N off the multiples of 8 (C rows at any alignment): split
 # sums, whole tiles, K a multiple of 8 or not, fewer than 16 columns
-COPIES = [(300, 201, 4095), (129, 9, 4097), (700, 700, 11273), (2049, 2051, 2052), (4096, 4095, 1032), (4000, 4001, 33),
+COPIES = [(300, 201, 4095), (129, 9, 4097), (500, 500, 12297), (2049, 2051, 2052), (4096, 4095, 1032), (4000, 4001, 33),
           (4000, 4003, 40)]
 
 

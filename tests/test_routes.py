@@ -66,18 +66,32 @@ def test_odd_k_of_few_rows(kernel, call, name):
 # version 15 through registers or through copies and version 10
 @pytest.mark.parametrize("call,name", [
     ((F16, 15, 1000, 1001, 999), "f16_any"),
-    ((F16, 15, 700, 700, 11263), "f16_any"),       # few tiles: odd K up to 11264
-    ((F16, 15, 700, 700, 11265), "f16_pp16"),
-    ((F16, 15, 700, 700, 14332), "f16_any"),       # even K up to 14336
-    ((F16, 15, 700, 700, 14338), "f16_pp16"),
-    ((F16, 15, 700, 701, 12288), "f16_any"),       # K a multiple of 8 up to 12288
-    ((F16, 15, 700, 701, 12296), "f16_pp16"),
+    ((F16, 15, 500, 500, 12287), "f16_any"),       # few tiles: odd K up to 12288
+    ((F16, 15, 500, 500, 12289), "f16_pp16"),
+    ((F16, 15, 700, 700, 16385), "f16_any"),       # and 8 tiles of 256 x 256
+    ((F16, 15, 5825, 33, 14805), "f16_any"),
+    ((F16, 15, 500, 500, 16382), "f16_any"),       # even K up to 16384
+    ((F16, 15, 500, 500, 16386), "f16_pp16"),
+    ((F16, 15, 1987, 128, 17674), "f16_any"),
+    ((F16, 15, 13398, 30, 17198), "f16_any"),
+    ((F16, 15, 700, 697, 13312), "f16_any"),       # K a multiple of 8 up to 13312
+    ((F16, 15, 700, 697, 13320), "f16_pp16"),
+    ((F16, 15, 697, 700, 13320), "f16_any"),       # N up to M
+    ((F16, 15, 14946, 29, 14024), "f16_any"),
     ((F16, 15, 300, 200, 1023), "f16_any"),        # fewer still: K up to 1024
     ((F16, 15, 300, 200, 4095), "f16_pp16"),
     ((F16, 15, 1000, 2001, 4096), "f16_any"),      # more tiles than CUs
-    ((F16, 15, 10000, 101, 6144), "f16_pp16"),
-    ((F16, 15, 8000, 257, 2048), "f16_any"),       # two per CU
-    ((F16, 15, 8000, 257, 3072), "f16_pp16"),
+    ((F16, 15, 2461, 411, 4608), "f16_any"),
+    ((F16, 15, 2461, 411, 4616), "f16_pp16"),
+    ((F16, 15, 2461, 412, 6144), "f16_any"),       # rows of B that start on dwords
+    ((F16, 15, 2461, 412, 6152), "f16_pp16"),
+    ((F16, 15, 413, 2535, 5584), "f16_any"),       # N above 2 M
+    ((F16, 15, 2764, 365, 6144), "f16_any"),       # more than 21 of 256 x 256
+    ((F16, 15, 2764, 365, 6152), "f16_pp16"),
+    ((F16, 15, 365, 2764, 6152), "f16_any"),
+    ((F16, 15, 16567, 35, 14450), "f16_any"),      # both copied
+    ((F16, 15, 8000, 257, 3072), "f16_any"),       # two per CU
+    ((F16, 15, 763, 3761, 2696), "f16_any"),
     ((F16, 15, 128, 50001, 1023), "f16_any"),      # half-empty 256 x 256 tiles
     ((F16, 15, 100000, 65, 513), "f16_any"),
     ((F16, 15, 100000, 65, 512), "f16_pp16"),
@@ -90,9 +104,19 @@ def test_odd_k_of_few_rows(kernel, call, name):
     ((F16, 15, 16000, 401, 512), "f16_pp16"),      # only B copied
     ((F16, 15, 236, 16964, 1024), "f16_any"),      # and its rows start on dwords
     ((F16, 15, 512, 4978, 3368), "f16_any"),
-    ((F16, 15, 512, 4979, 2568), "f16_pp16"),
-    ((F16, 15, 3000, 1500, 1500), "f16_any"),      # even K
-    ((F16, 15, 3000, 1500, 1025), "f16_pp16"),
+    ((F16, 15, 400, 15001, 512), "f16_any"),       # few rows
+    ((F16, 15, 401, 15001, 264), "f16_pp16"),
+    ((F16, 15, 3000, 1500, 1700), "f16_any"),      # even K
+    ((F16, 15, 3000, 1500, 1281), "f16_pp16"),
+    ((F16, 15, 3000, 1500, 1279), "f16_any"),
+    ((F16, 15, 384, 14001, 1401), "f16_any"),      # narrow
+    ((F16, 15, 14001, 384, 1401), "f16_any"),
+    ((F16, 15, 14001, 385, 1401), "f16_pp16"),
+    ((F16, 15, 11118, 1328, 21), "f16_any"),       # small K, one residency
+    ((F16, 15, 281, 41448, 46), "f16_any"),
+    ((F16, 15, 11118, 1328, 129), "f16_pp16"),
+    ((F16, 15, 239, 74678, 144), "f16_any"),       # few rows
+    ((F16, 15, 239, 74679, 144), "f16_pp16"),
     ((F16, 15, 50000, 305, 64), "f16_pp16"),
     ((F16, 15, 300, 50001, 130), "f16_any"),
     ((F16, 15, 1000, 8001, 1023), "f16_any"),      # two 128 x 128 tiles per CU

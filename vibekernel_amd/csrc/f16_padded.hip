@@ -128,28 +128,35 @@ bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_str
 //    182 / 140, x 96 16.5 / 22, 300000 x 2 x 128 59 / 48, 46840 x 1 x 688 60 / 26; 20000 x
 //    3 x 256 9.8 / 13.8, 2000 x 1 x 688 16.8 / 20.7, x 1024 26.4 / 25.9;
 //  * while 64 x 64 tiles are at most 4 per CU (f16_any_launch's rule for them): 1000
-//    x 1001 x 1023 13.0 / 34.3, 2000 x 2001 x 2001 48 / 55; but a workgroup's
-//    k-loop is one chain, which the copies' split sum cuts in 8: 224 x 968 x 10242
-//    48 / 64, x 14340 70 / 75, x 16380 85 / 80; odd K, whose rows of A straddle dwords,
-//    224 x 968 x 10241 64 / 64, 700 x 700 x 11267 66 / 72, 1000 x 136 x 11267 68 / 66,
-//    200 x 500 x 32767 215 / 129; B alone copied, 224 x 969 x 12288 61 / 68, x 14336 75
-//    / 72, with more tiles than CUs 10000 x 101 x 4096 48 / 46, 1000 x 2001 x 4096 40 /
-//    48, with two per CU 8000 x 257 x 2048 36 / 45, x 3072 51 / 43, 512 x 4978 x 2624 38
-//    / 47.  Fewer tiles than an
-//    eighth of the CUs keep version 10's split sum (and its bits) from K = 1025 on,
-//    though 300 x 200 x 4095 takes 28.7 / 49;
+//    x 1001 x 1023 13.0 / 34.3, 2000 x 2001 x 2001 48 / 55.  But a workgroup's k-loop
+//    is one chain there.  Few 256 x 256 tiles, which the copies' sum splits 8 or 12 to
+//    32 ways, win a deep enough K, unless most of them is empty or copies of a wide
+//    B are most of the work: up to a tile per CU, B alone copied, 779 x 148 x 13032
+//    61 / 65, 2845 x 67 x 14536 85 / 75, 218 x 2606 x 12448 68 / 90, 14946 x 29 x 14024
+//    97 / 131; odd K, whose rows of A straddle dwords, 361 x 418 x 11377 66 / 68, 245 x
+//    1272 x 14363 92 / 78, 5825 x 33 x 14805 102 / 154; even K 238 x 1456 x 14678 83 / 80,
+//    141 x 852 x 14366 66 / 74, 1085 x 178 x 19398 120 / 94, 1987 x 32 x 17674 84 / 97,
+//    13398 x 30 x 17198 100 / 314.  With more tiles, B alone copied, 2463 x 419 x 7744
+//    68 / 55, 2332 x 409 x 5776 52 / 52, 2764 x 365 x 8104 76 / 63, 413 x 2535 x 5584
+//    54 / 62, 763 x 3761 x 2696 43 / 56; with A too 22016 x 16 x 18286 188 / 547.  Fewer
+//    tiles than an eighth of the CUs keep version 10's split sum (and its bits) from
+//    K = 1025 on, though 300 x 200 x 4095 takes 28.7 / 49;
 //  * where half of each 256 x 256 tile is empty: 128 x 50001 x 1023 53 / 67, 100000
 //    x 65 x 513 63 / 79, but 100000 x 65 x 512 56 / 42, x 256 35 / 31;
-//  * while 128 x 128 tiles are at most 2 per CU, up to K = 1024, or 1536 even: 1000 x
-//    8001 x 129 18.4 / 20.4, 3000 x 1500 x 1023 35 / 40, x 1500 43 / 46, 1500 x 3001 x
-//    1801 63 / 52; B alone copied, 16000 x 401 x 512 24.7 / 20.2, 236 x 16964 x 1024 36
-//    / 43;
+//  * while 128 x 128 tiles are at most 2 per CU, even K and narrow products: 1000 x
+//    8001 x 129 18.4 / 20.4, 3000 x 1500 x 1023 35 / 40, x 1500 43 / 46, 26144 x 138 x
+//    1910 67 / 80, 3056 x 1576 x 1690 47 / 48, 7627 x 516 x 2126 60 / 67, 19652 x 262 x
+//    1461 56 / 62, but 4326 x 1473 x 1281 51 / 43; B alone copied 16000 x 401 x 512 24.7 / 20.2, 226 x 21777 x
+//    488 26 / 28, 221 x 30095 x 832 38 / 44;
+//  * small K while 128 x 128 tiles are one residency there (4 per CU) and 256 x 256
+//    tiles more than one: 11118 x 1328 x 21 16.9 / 19.9, 281 x 41448 x 46 17.8 / 21.9;
 //  * past that few columns up to K = 256, whose copy of A is most of the work:
 //    50000 x 304 x 193 32 / 36, x 257 47 / 43, 50000 x 200 x 193 24 / 29, x 385 45 /
 //    39, 30000 x 600 x 129 28.0 / 29.6; 50000 x 400 x 65 28.7 / 26.3; and few rows whose
 //    A or B starts on dwords: 300 x 50000 x 193 32 / 35, x 257 47 / 40; 300 x 50001 x 65
 //    30.3 / 29.5, x 130 28.6 / 31.8; 400 x 50000 x 65 31.5 / 26.3, 129 x 100000 x 129
-//    38.7 / 34.0;
+//    38.7 / 34.0; 220 x 42640 x 155 20.6 / 22.9, 239 x 74678 x 144 29.8 / 33.7, 161 x
+//    55546 x 16 15.7 / 12.5;
 //  * the rest take the copies: 4000 x 4000 x 33 18.6 / 15.3, 4096 x 8192 x 255 55 /
 //    40, 8192 x 8193 x 65 111 / 59.
 bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
@@ -159,19 +166,34 @@ bool no_copies(size_t m, size_t n, size_t k, int num_cus) {
   const size_t c = num_cus;
   const bool copy_a = k % 8 != 0;
   auto tiles = [&](size_t t) { return (m + t - 1) / t * ((n + t - 1) / t); };
-  const size_t small = tiles(64);
+  const size_t small = tiles(64), tiles256 = tiles(256);
   if (n < 8) return k <= (copy_a ? 384 : 120) || (k <= 768 && m * k < (size_t)1 << 23);
   if (small <= 4 * c) {
-    size_t deepest = k % 2 ? 11264 : copy_a ? 14336 : small <= c ? 12288 : small <= 2 * c ? 4608 : 2560;
-    if (n % 2 == 0 && !copy_a && small > c) deepest += 1536;  // B's rows start on dwords
-    return k <= 1024 || (8 * small >= c && k <= deepest);
+    if (k <= 1024) return true;
+    if (8 * small < c) return false;
+    bool copies;
+    if (copy_a)
+      copies = small <= c && 32 * tiles256 <= c && (k % 2 ? k > 12288 : k > 16384 && std::min(m, n) > 128);
+    else if (small <= c)
+      copies = k > 13312 && n <= m && 20 * tiles256 <= c;
+    else if (12 * tiles256 <= c)
+      copies = k > (n % 2 ? 4608 : 6144) && n <= 2 * m;  // even N: B's rows start on dwords
+    else
+      copies = k > 6144 && n <= m && 10 * tiles256 <= c;
+    return !copies;
   }
   if (m <= 128) return true;
   if (n <= 128) return copy_a || k < 256;
-  if (tiles(128) <= 2 * c) return k <= (!copy_a && n % 2 ? 256 : k % 2 ? 1024 : 1536);
+  const size_t tiles128 = tiles(128);
+  if (tiles128 <= 2 * c) {
+    if (copy_a) return k % 2 == 0 || k <= 1280 || std::min(m, n) <= 384;
+    return m <= 400 || k <= (n % 2 ? 256 : 1536);
+  }
+  if (tiles128 <= 4 * c && tiles256 > c && k <= 128) return true;
+  const bool few = tiles128 <= 5 * c;
+  if (few && m <= 256 && n % 2 == 0 && k > 40 && k <= 256) return true;
   if (!copy_a || k > 256) return false;
-  const size_t filled = 100 * m * n / (tiles(256) * 65536);  // per cent of the 256 x 256 tiles
-  const bool few = tiles(128) <= 5 * c;
+  const size_t filled = 100 * m * n / (tiles256 * 65536);  // per cent of the 256 x 256 tiles
   return m > n ? n <= 256 || filled <= (few ? 80 : 60) : (n % 8 == 0 || k % 2 == 0) && k > 64 && filled <= 60 && few;
 }
 
