@@ -54,9 +54,11 @@ def test_wide_tiles_of_version_11(kernel, call, wide):
     assert ("f16_pp128n_kernel" in name and "ELb0ELb1EE" in name) == wide, name
 
 
-# few rows of version 15: A by whole dwords where K is odd (the last template argument)
+# few rows of version 15: A by whole dwords where K is odd and M above 9 (the last template argument)
 @pytest.mark.parametrize("call,name", [((F16, 15, 16, 4095, 4096), "f16_stream_kernelILi1EDF16_Lb0EE"),
                                        ((F16, 15, 16, 4095, 4095), "f16_stream_kernelILi1EDF16_Lb1EE"),
+                                       ((F16, 15, 10, 4095, 4095), "f16_stream_kernelILi1EDF16_Lb1EE"),
+                                       ((F16, 15, 9, 4095, 4095), "f16_stream_kernelILi1EDF16_Lb0EE"),
                                        ((F16, 15, 128, 4096, 4094), "f16_stream_kernelILi4EDF16_Lb0EE"),
                                        ((F16, 15, 128, 4096, 4095), "f16_stream_kernelILi4EDF16_Lb1EE")])
 def test_odd_k_of_few_rows(kernel, call, name):

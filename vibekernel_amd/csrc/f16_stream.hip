@@ -21,7 +21,7 @@
 //    bytes per load); kD k-steps of both are in flight per wave.  Where K is
 //    odd, every other row starts between two dwords, and such loads from 16
 //    rows take half as long again as B's: A is then loaded by whole dwords,
-//    one more per fragment, and shifted;
+//    one more per fragment, and shifted (up to 9 rows as it is);
 //  * the lanes of a last column block that N cuts short take the last 8
 //    columns of the matrix instead (N >= 8): every load stays inside B, and
 //    columns computed twice are the same sum stored twice;
@@ -42,7 +42,8 @@
 // 16 x 4095 x 4096 13.8 against 59; 64 x 1001 x 1025 15.5 against 33.5; 16 x
 // 301 x 16000 14.5 against 74.  Odd K, with A shifted in registers and as loaded
 // before: 16 / 64 / 128 x 16391 x 4095 40.5 / 59.7 / 92.6 and 43.2 / 78.0 / 141
-// (copies: 127); 128 x 50256 x 1025 62.9 and 82.3 (65.5).
+// (copies: 127); 128 x 50256 x 1025 62.9 and 82.3 (65.5); 15 x 4816 x 9409 27.7 and
+// 28.5, but 9 x 3920 x 5637 15.6 and 15.2, 3 x 3584 x 1183 7.5 and 7.2.
 #include "vk_device.hpp"
 #include "vk_internal.hpp"
 #include "vk_stream.hpp"
@@ -272,7 +273,7 @@ hipError_t launch_out(const GemmArgs& a, size_t ws_limit) {
 }
 template <int MB>
 hipError_t launch_mb(const GemmArgs& a, size_t ws_limit) {
-  return a.k % 2 && a.m > 1 ? launch_out<MB, true>(a, ws_limit) : launch_out<MB, false>(a, ws_limit);
+  return a.k % 2 && a.m > 9 ? launch_out<MB, true>(a, ws_limit) : launch_out<MB, false>(a, ws_limit);
 }
 
 }  // namespace
