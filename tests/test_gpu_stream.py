@@ -76,8 +76,9 @@ def test_repeats_and_shared_workspace(gpu):
 
 # K one past the whole 32-deep steps: the last element of A ends the last
 # fragment's dword where the last row is odd, and is past it where it is even
-@pytest.mark.parametrize("shape", [(1, 40, 1025), (2, 40, 1025), (11, 40, 1025), (16, 40, 1025), (31, 136, 1057), (32, 136, 1057), (47, 264, 2049),
-                                   (64, 264, 2049), (95, 129, 1089), (96, 129, 1089), (127, 72, 4129), (128, 72, 4129)])
+@pytest.mark.parametrize("shape", [(1, 40, 1025), (2, 40, 1025), (11, 40, 1025), (16, 40, 1025), (31, 136, 1057),
+                                   (32, 136, 1057), (47, 264, 2049), (64, 264, 2049), (95, 129, 1089), (96, 129, 1089),
+                                   (127, 72, 4129), (128, 72, 4129)])
 def test_odd_k(gpu, shape):
     m, n, k = shape
     A, B = make_inputs(m, n, k, "int", seed=m + n + k)
