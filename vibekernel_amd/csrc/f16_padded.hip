@@ -129,9 +129,9 @@ bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_str
 //    3 x 256 9.8 / 13.8, 2000 x 1 x 688 16.8 / 20.7, x 1024 26.4 / 25.9;
 //  * while 64 x 64 tiles are at most 4 per CU (f16_any_launch's rule for them): 1000
 //    x 1001 x 1023 13.0 / 34.3, 2000 x 2001 x 2001 48 / 55.  But a workgroup's k-loop
-//    is one chain there.  Few 256 x 256 tiles, which the copies' sum splits 8 or 12 to
-//    32 ways, win a deep enough K, unless most of them is empty or copies of a wide
-//    B are most of the work: up to a tile per CU, B alone copied, 779 x 148 x 13032
+//    is one chain there, and version 10 splits the sum of few 256 x 256 tiles 10 to 32
+//    ways or more: the copies win a deep enough K, unless most of those tiles is empty
+//    or copying a wide B is most of the work: up to a tile per CU, B alone copied, 779 x 148 x 13032
 //    61 / 65, 2845 x 67 x 14536 85 / 75, 218 x 2606 x 12448 68 / 90, 14946 x 29 x 14024
 //    97 / 131; odd K, whose rows of A straddle dwords, 361 x 418 x 11377 66 / 68, 245 x
 //    1272 x 14363 92 / 78, 5825 x 33 x 14805 102 / 154; even K 238 x 1456 x 14678 83 / 80,
@@ -146,8 +146,8 @@ bool few_rows(size_t m, size_t n, size_t k) { return (n % 8 || k % 8) && f16_str
 //  * while 128 x 128 tiles are at most 2 per CU, even K and narrow products: 1000 x
 //    8001 x 129 18.4 / 20.4, 3000 x 1500 x 1023 35 / 40, x 1500 43 / 46, 26144 x 138 x
 //    1910 67 / 80, 3056 x 1576 x 1690 47 / 48, 7627 x 516 x 2126 60 / 67, 19652 x 262 x
-//    1461 56 / 62, but 4326 x 1473 x 1281 51 / 43; B alone copied 16000 x 401 x 512 24.7 / 20.2, 226 x 21777 x
-//    488 26 / 28, 221 x 30095 x 832 38 / 44;
+//    1461 56 / 62, but 4326 x 1473 x 1281 51 / 43; B alone copied 16000 x 401 x 512
+//    24.7 / 20.2, 226 x 21777 x 488 26 / 28, 221 x 30095 x 832 38 / 44;
 //  * small K while 128 x 128 tiles are one residency there (4 per CU) and 256 x 256
 //    tiles more than one: 11118 x 1328 x 21 16.9 / 19.9, 281 x 41448 x 46 17.8 / 21.9;
 //  * past that few columns up to K = 256, whose copy of A is most of the work:
